@@ -445,13 +445,31 @@ __device__ __forceinline__ uint2 get_codes(const void *__restrict__ bkt, uint64_
     }
 }
 
+// Pass 1 sorts by the coarse bucket and the top J bits of the fine index
+// (rows of pass 1: B << J per set); pass 2 sorts each row by the remaining s1
+// bits.  A pass's counters, ballots and piece lengths go with its own bucket
+// count (50 Mbp job, 64 x 512 buckets, the two scatters: 6 + 9 bits 529 + 515 us,
+// 7 + 8 bits 553 + 448, 8 + 7 bits 615 + 387).
+// A k-mer's code is its fine bucket in slot order: coarse bucket above, fine
+// index below, the fine index of a set with fewer than J fine bits moved up
+// (the rows between stay empty), so row = code >> s1 and equal codes are equal
+// fine buckets.
+__host__ __device__ constexpr uint32_t split_bits(uint32_t sb, uint32_t J)
+{
+    return (sb > J ? sb : J) | (sb < J ? J - sb : 0u) << 8 | (sb > J ? sb - J : 0u) << 16;
+}
+__device__ __forceinline__ uint32_t split_code(uint32_t f, uint32_t bmask, uint32_t nbits, uint32_t split)
+{
+    return (f & bmask) << (split & 0xFFu) | (f >> nbits) << ((split >> 8) & 0xFFu);
+}
+
 template <int W, int IPT, int MODE, bool C32>
 __global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict__ kin, const BTile *__restrict__ tiles,
-                                                      LminParams p, uint64_t top_mask, void *__restrict__ bkt,
-                                                      uint32_t *__restrict__ hist, uint32_t *__restrict__ xhist,
-                                                      uint32_t n_tiles)
+                                                      LminParams p, uint32_t R, uint64_t top_mask,
+                                                      void *__restrict__ bkt, uint32_t *__restrict__ hist,
+                                                      uint32_t *__restrict__ xhist, uint32_t n_tiles)
 {
-    extern __shared__ uint32_t cnt[];  // B buckets + 1 crossing counter
+    extern __shared__ uint32_t cnt[];  // R rows + 1 crossing counter
     // (XCD-contiguous tiles: neighbouring tiles write neighbouring words of
     // every bucket's histogram row, which one L2 then merges into whole lines)
     const uint32_t ti = xcd_tile(n_tiles);
@@ -460,9 +478,9 @@ __global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict
     // fine bucket = order & (B*S - 1); its low log2(B) bits are the coarse
     // bucket.  A k-mer crosses when its two fine buckets differ (both copies
     // may then share a coarse bucket).
-    for (uint32_t i = threadIdx.x; i <= p.B; i += BLOCK) cnt[i] = 0;
+    for (uint32_t i = threadIdx.x; i <= R; i += BLOCK) cnt[i] = 0;
     __syncthreads();
-    const uint32_t bmask = p.B - 1;
+    const uint32_t bmask = p.B - 1, nbits = (uint32_t)__builtin_ctz(p.B), s1 = t.split >> 16;
     // all of this thread's k-mers in flight at once
     Kmer<W> xs[IPT];
 #pragma unroll
@@ -476,17 +494,18 @@ __global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict
         if (idx >= t.count) continue;
         uint32_t o1, o2;
         double_lmin<W, MODE>(xs[j], p, o1, o2);
-        const uint32_t f1 = o1 & t.fmask, f2 = o2 & t.fmask;
+        const uint32_t f1 = split_code(o1 & t.fmask, bmask, nbits, t.split);
+        const uint32_t f2 = split_code(o2 & t.fmask, bmask, nbits, t.split);
         put_codes<C32>(bkt, t.kbegin + idx, f1, f2);
-        atomicAdd(&cnt[f1 & bmask], 1u);
+        atomicAdd(&cnt[f1 >> s1], 1u);
         if (f1 != f2) {
-            atomicAdd(&cnt[f2 & bmask], 1u);
-            atomicAdd(&cnt[p.B], 1u);
+            atomicAdd(&cnt[f2 >> s1], 1u);
+            atomicAdd(&cnt[R], 1u);
         }
     }
     __syncthreads();
-    for (uint32_t b = threadIdx.x; b < p.B; b += BLOCK) hist[t.hbase + (uint64_t)b * t.ts + t.tlocal] = cnt[b];
-    if (threadIdx.x == 0) xhist[ti] = cnt[p.B];
+    for (uint32_t b = threadIdx.x; b < R; b += BLOCK) hist[t.hbase + (uint64_t)b * t.ts + t.tlocal] = cnt[b];
+    if (threadIdx.x == 0) xhist[ti] = cnt[R];
 }
 
 // lanes whose home (mp) or borrow (ms) placement goes to bucket v
@@ -670,6 +689,7 @@ __global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict_
     const uint32_t ti = xcd_tile(n_tiles);
     if (ti == NONE) return;
     const BTile t = tiles[ti];
+    const uint32_t s1 = t.split >> 16;
     // all of this thread's codes and k-mers in flight at once
     uint2 codes[IPT];
     Kmer<W> xs[IPT];
@@ -710,8 +730,8 @@ __global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict_
         uint32_t bp = 0, bs = 0;
         bool cross = false;
         if (valid) {
-            bp = codes[j].x & (B - 1);
-            bs = codes[j].y & (B - 1);
+            bp = codes[j].x >> s1;
+            bs = codes[j].y >> s1;
             cross = codes[j].x != codes[j].y;
         }
         const uint64_t V = __ballot(valid), C = __ballot(cross);
@@ -768,8 +788,8 @@ __global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict_
         if (idx >= t.count) continue;
         const uint64_t g = t.kbegin + idx;
         const uint2 c = codes[j];
-        const uint32_t fp = c.x >> nbits, fs = c.y >> nbits;  // fine indices inside the coarse buckets
-        const uint32_t bp = c.x & (B - 1), bs = c.y & (B - 1);
+        const uint32_t bp = c.x >> s1, bs = c.y >> s1;
+        const uint32_t fp = c.x & ((1u << s1) - 1u), fs = c.y & ((1u << s1) - 1u);  // fine indices inside the rows
         const bool cross = c.x != c.y;
         const uint16_t *gc = gcnt + (size_t)(j * NW + w) * (B + 1);
         const Kmer<W> x = xs[j];
@@ -824,10 +844,10 @@ __global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict_
 
 // pass-1 tiles from the per-set plan: set s owns tiles [tfirst[s],
 // tfirst[s + 1]) (at least one, possibly empty, so that every bucket row has
-// a start in the histogram) and histogram entries from B * tfirst[s]
+// a start in the histogram) and histogram entries from (B << J) * tfirst[s]
 __global__ void k_plan1_tiles(const uint64_t *__restrict__ set_off, const uint64_t *__restrict__ tfirst,
-                              const uint32_t *__restrict__ set_sub, uint32_t n_sets, uint32_t B, uint32_t tile,
-                              uint64_t T, BTile *__restrict__ tiles)
+                              const uint32_t *__restrict__ set_sub, uint32_t n_sets, uint32_t B, uint32_t J,
+                              uint32_t tile, uint64_t T, BTile *__restrict__ tiles)
 {
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= T) return;
@@ -840,42 +860,48 @@ __global__ void k_plan1_tiles(const uint64_t *__restrict__ set_off, const uint64
     const uint64_t ns = set_off[lo + 1] - set_off[lo], tl = t - tfirst[lo], skip = tl * tile;
     BTile bt;
     bt.kbegin = set_off[lo] + skip;
-    bt.hbase = (uint64_t)B * tfirst[lo];
+    bt.hbase = (uint64_t)(B << J) * tfirst[lo];
     bt.count = (uint32_t)(ns > skip ? (ns - skip < tile ? ns - skip : tile) : 0);
     bt.set = lo;
     bt.ts = (uint32_t)(tfirst[lo + 1] - tfirst[lo]);
     bt.tlocal = (uint32_t)tl;
     bt.fmask = B * set_sub[lo] - 1;
-    bt.pad = 0;
+    bt.split = split_bits((uint32_t)__builtin_ctz(set_sub[lo]), J);
     tiles[t] = bt;
 }
 
-// bucket row starts: boff[set*B + b] = scanned histogram at the set's first tile
-// (and the same rows into boff2 when given: the fine rows of a job without
-// a fine sort).  The slot count is *mdev when given (the host has not read
-// it), else m.
+// row starts: rows[set * (B << J) + row] = scanned histogram at the set's
+// first tile; a coarse bucket begins at its first row (boff), and without a
+// second pass a fine bucket is its row (fboff, when given; row_first[r + 1] >
+// row_first[r] for the rows that are one).  The slot count is *mdev when
+// given (the host has not read it), else m.
 __global__ void k_gather_boff(const uint32_t *__restrict__ hscan, const uint64_t *__restrict__ set_hbase,
-                              const uint32_t *__restrict__ set_ts, uint32_t n_sets, uint32_t B, uint32_t m,
-                              const uint32_t *__restrict__ mdev, uint32_t *__restrict__ boff,
-                              uint32_t *__restrict__ boff2)
+                              const uint32_t *__restrict__ set_ts, uint32_t n_sets, uint32_t R, uint32_t J, uint32_t m,
+                              const uint32_t *__restrict__ mdev, const uint32_t *__restrict__ row_first,
+                              uint32_t *__restrict__ rows, uint32_t *__restrict__ boff, uint32_t *__restrict__ fboff)
 {
     const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t G = n_sets * B;
+    const uint32_t G = n_sets * R;
     uint32_t v;
     if (g < G) {
-        const uint32_t s = g / B, b = g % B;
+        const uint32_t s = g / R, b = g % R;
         v = hscan[set_hbase[s] + (uint64_t)b * set_ts[s]];
     } else if (g == G) {
         v = mdev ? *mdev : m;
     } else {
         return;
     }
-    boff[g] = v;
-    if (boff2) boff2[g] = v;
+    rows[g] = v;
+    if (boff && !(g & ((1u << J) - 1u))) boff[g >> J] = v;
+    if (fboff) {
+        const uint32_t f = row_first[g];
+        if (g == G || row_first[g + 1] > f) fboff[f] = v;
+    }
 }
 
-// ---- fine buckets: a stable counting sort of every coarse bucket's slots by
-// their fine index (the next bits of the same minimizer order)
+// ---- fine buckets: a stable counting sort of every pass-1 row's slots by
+// the rest of their fine index (the next bits of the same minimizer order);
+// "coarse bucket" below is such a row
 
 // Pass-2 tiles are planned on the device from the coarse rows: coarse
 // bucket g (S_g fine buckets, ts_g = max(1, ceil(rows / tile)) tiles) owns
@@ -946,7 +972,7 @@ __global__ void k_plan2_tiles(const uint32_t *__restrict__ boff, const uint32_t 
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_tiles) return;
     BTile bt;
-    bt.pad = 0;
+    bt.split = 0;
     if (i >= cb_tfirst[G]) {
         bt.kbegin = 0;
         bt.hbase = 0;
@@ -2843,7 +2869,7 @@ struct uc_ctx {
         cbfirst, fboff, egroups, fbbase, scan_tmp, kmer, flags, src, pair_h, pair_b, boff, etiles,
         toff, tcap, table, hit, link, hasp, pred, seg, prevseg, chainA, chainB, cycB, list, clist, ulen, tsum,
         htoff, setoff, text, small, txt, txtcnt, rec, rch, tcnt, cbtf, over, colsum, bgroups, gfirst, stasks,
-        mlist, mcnt, probes;
+        mlist, mcnt, probes, rows;
     // pinned host chunks of the file reader and writer
     // pinned bounce buffer of the small device reads (counters, offsets):
     // a copy into pinned memory completes sooner than one into pageable
@@ -2919,7 +2945,7 @@ static std::vector<DBuf *> all_bufs(uc_ctx *c)
             &c->cycB,   &c->list,    &c->clist,  &c->ulen,    &c->tsum,    &c->htoff,  &c->setoff,
             &c->text,   &c->small,   &c->txt,    &c->txtcnt,  &c->rec,     &c->rch,
             &c->tcnt,   &c->cbtf,    &c->over,   &c->colsum, &c->bgroups, &c->gfirst, &c->stasks,
-            &c->mlist,  &c->mcnt,    &c->probes};
+            &c->mlist,  &c->mcnt,    &c->probes,  &c->rows};
 }
 
 static void free_pinned(uc_ctx *c)
@@ -3827,6 +3853,23 @@ int check_placements(uc_ctx *c, uint64_t n, uint64_t x)
 
 constexpr uint64_t FINE_CAPPED_MAX = 1700;
 
+// fine bits that pass 1 takes (see split_bits): all of them when the fine
+// buckets are at most MAX_BUCKETS (no second pass: seven launches fewer, 100 k
+// 63-mers 231 -> 210 us), else one less than half of all bits with the coarse
+// ones (50 Mbp 31-mers, 6 + 9 bits 1536 us of bucketing, 7 + 8 1525, 8 + 7 1531,
+// 9 + 6 1778; 12 M 47-mers, 6 + 10 bits 597, 7 + 9 566, 8 + 8 573, 9 + 7 633).
+// A batch of many sets keeps the rows of all sets few enough for the host to
+// plan.
+static uint32_t pass1_fine_bits(uint32_t nb, uint32_t sb, uint32_t n_sets)
+{
+    constexpr uint32_t most = 10;  // log2 MAX_BUCKETS
+    static_assert(1u << most == MAX_BUCKETS, "pass 1 ranks up to MAX_BUCKETS rows");
+    const uint32_t half = (nb + sb - 1) / 2;
+    uint32_t J = nb + sb <= most ? sb : half > nb ? std::min(half, most) - nb : 0;
+    while (J && ((uint64_t)n_sets << (nb + J)) > 65536) J--;
+    return J;
+}
+
 template <int W>
 int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
 {
@@ -3835,7 +3878,6 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     // fine buckets per coarse bucket, per set: about FINE_TARGET slots each
     const uint64_t fine_target = c->opts.fine_slots ? c->opts.fine_slots : (W_ == 1 ? 512 : 384);
     c->set_sub.assign(S, 1);
-    bool any_fine = false;
     for (uint32_t s = 0; s < S; s++) {
         const uint64_t ns = c->set_off[s + 1] - c->set_off[s];
         const uint64_t want = (ns * 112 / 100 + (uint64_t)B * fine_target - 1) / ((uint64_t)B * fine_target);
@@ -3851,10 +3893,17 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         if (!c->opts.fine_slots && want > MAX_SUB && c->opts.mode != UC_MODE_PLAIN)
             while (sub > 1 && ns * 112 / 100 <= (uint64_t)B * (sub / 2) * FINE_CAPPED_MAX) sub >>= 1;
         c->set_sub[s] = sub;
-        any_fine |= sub > 1;
     }
     const bool keep_src = (c->opts.flags & UC_FLAG_KEEP_SRC) != 0;
     c->tile2 = 0;
+    // how the fine bits are split over the two passes (see split_bits)
+    const uint32_t nb = (uint32_t)__builtin_ctz(B);
+    uint32_t smax = 1;
+    for (uint32_t sb : c->set_sub) smax = std::max(smax, sb);
+    const uint32_t J = pass1_fine_bits(nb, (uint32_t)__builtin_ctz(smax), S);
+    const uint32_t R = B << J;                                    // pass-1 rows per set
+    const uint32_t s1max = std::max(smax >> J, 1u);               // most fine buckets of a row
+    const bool any_fine = s1max > 1;                              // a second pass follows
     // k-mers per bucketing tile
     constexpr int IPT1 = W == 1 ? 8 : 4;
     const uint32_t tile1 = IPT1 * BLOCK;
@@ -3870,7 +3919,7 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         const uint32_t ts = (uint32_t)std::max<uint64_t>(1, (ns + tile1 - 1) / tile1);
         set_plan[s] = c->set_off[s];
         set_plan[S + 1 + s] = T;
-        set_hbase[s] = (uint64_t)B * T;
+        set_hbase[s] = (uint64_t)R * T;
         set_ts[s] = ts;
         T += ts;
     }
@@ -3878,17 +3927,28 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     set_plan[2 * (uint64_t)S + 1] = T;
     uint32_t *sub_h = reinterpret_cast<uint32_t *>(set_plan.data() + 2 * (uint64_t)S + 2);
     for (uint32_t s = 0; s < S; s++) sub_h[s] = c->set_sub[s];
-    const uint64_t hb = (uint64_t)B * T;
-    const uint64_t G = (uint64_t)S * B;
+    const uint64_t hb = (uint64_t)R * T;
+    const uint64_t G = (uint64_t)S * B, GR = (uint64_t)S * R;
     // every coarse bucket's first fine bucket (from the sets' fine counts)
     c->cb_first.assign(G + 1, 0);
     for (uint64_t g = 0; g < G; g++) c->cb_first[g + 1] = c->cb_first[g] + c->set_sub[g / B];
     const uint64_t F = c->cb_first[G];
     // the host's plan in one upload, in 8-byte words: the coarse buckets'
     // first fine buckets (G + 1 u32), the set plan, the sets' histogram bases
-    // (u64) and tile counts (u32); cbfirst lives on to emission
-    const uint64_t w_cbf = (G + 2) / 2, w_plan = set_plan.size(), w_hb = S, w_ts = (S + 1) / 2;
-    std::vector<uint64_t> up(w_cbf + w_plan + w_hb + w_ts, 0);
+    // (u64) and tile counts (u32), with J > 0 the rows' first fine buckets
+    // (GR + 1 u32); cbfirst lives on to emission
+    const uint64_t w_cbf = (G + 2) / 2, w_plan = set_plan.size(), w_hb = S, w_ts = (S + 1) / 2,
+                   w_row = J ? (GR + 2) / 2 : 0;
+    std::vector<uint64_t> up(w_cbf + w_plan + w_hb + w_ts + w_row, 0);
+    if (J) {
+        uint32_t *rf = reinterpret_cast<uint32_t *>(up.data() + w_cbf + w_plan + w_hb + w_ts);
+        for (uint64_t g = 0; g < G; g++) {
+            const uint32_t sb = (uint32_t)__builtin_ctz(c->set_sub[g / B]);
+            for (uint32_t q = 0; q < 1u << J; q++)  // (a set with fewer than J fine bits: its rows are spread out)
+                rf[(g << J) + q] = c->cb_first[g] + (sb >= J ? q << (sb - J) : (q + (1u << (J - sb)) - 1) >> (J - sb));
+        }
+        rf[GR] = (uint32_t)F;
+    }
     std::memcpy(up.data(), c->cb_first.data(), (G + 1) * 4);
     std::memcpy(up.data() + w_cbf, set_plan.data(), w_plan * 8);
     std::memcpy(up.data() + w_cbf + w_plan, set_hbase.data(), S * 8);
@@ -3898,9 +3958,10 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     const uint64_t *sp = P<uint64_t>(c->cbfirst) + w_cbf;
     const uint64_t *sethb = sp + w_plan;
     const uint32_t *setts = reinterpret_cast<const uint32_t *>(sethb + w_hb);
+    const uint32_t *row_first = J ? reinterpret_cast<const uint32_t *>(sethb + w_hb + w_ts) : P<uint32_t>(c->cbfirst);
     CHK(ensure(c, c->tiles, T * sizeof(BTile)));
     KLAUNCH(c, "k_plan1_tiles", k_plan1_tiles, (grid_for(T), BLOCK, 0), sp, sp + S + 1,
-            reinterpret_cast<const uint32_t *>(sp + 2 * (uint64_t)S + 2), S, B, tile1, T, P<BTile>(c->tiles));
+            reinterpret_cast<const uint32_t *>(sp + 2 * (uint64_t)S + 2), S, B, J, tile1, T, P<BTile>(c->tiles));
     CHK(ensure(c, c->hist, (hb + 1) * 4));
     CHK(ensure(c, c->xhist, (T + 1) * 4));
 
@@ -3919,14 +3980,12 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     p.table = table;
 
     const uint64_t *kin = c->kin;
-    // both fine codes of a k-mer in one word when every fine index fits 16 bits
-    uint32_t smax = 1;
-    for (uint32_t sb : c->set_sub) smax = std::max(smax, sb);
-    const bool c32 = (uint64_t)B * smax <= 65536;
+    // both fine codes of a k-mer in one word when every code fits 16 bits
+    const bool c32 = (uint64_t)R * s1max <= 65536;
     CHK(ensure(c, c->bkt, std::max<uint64_t>(c->n, 1) * (c32 ? 4 : 8)));
 #define UC_CNT(MODE, C32)                                                                                          \
-    KLAUNCH(c, "k_lmin_count", (k_lmin_count<W, IPT1, MODE, C32>), (xcd_grid(T), BLOCK, (B + 1) * 4), kin,        \
-            P<BTile>(c->tiles), p, c->top_mask, c->bkt.p, P<uint32_t>(c->hist), P<uint32_t>(c->xhist), tile_arg_xcd(T))
+    KLAUNCH(c, "k_lmin_count", (k_lmin_count<W, IPT1, MODE, C32>), (xcd_grid(T), BLOCK, (R + 1) * 4), kin,        \
+            P<BTile>(c->tiles), p, R, c->top_mask, c->bkt.p, P<uint32_t>(c->hist), P<uint32_t>(c->xhist), tile_arg_xcd(T))
     switch (lmin_mode(l, table != nullptr)) {
     case LM_TABLE:
         if (c32) { UC_CNT(LM_TABLE, true); } else { UC_CNT(LM_TABLE, false); }
@@ -3964,8 +4023,8 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         c->m = c->n + c->x;
         c->sizes_pending = false;
     }
-    // pass 1 writes the final k-mers and flags when no set is split into
-    // fine buckets, else the k-mers and the fine index with the flag bits
+    // pass 1 writes the final k-mers and flags when its rows are the fine
+    // buckets, else the k-mers and the rest of the fine index with the flag bits
     DBuf &k1 = any_fine ? c->kmer2 : c->kmer, &s1 = any_fine ? c->src2 : c->src;
     CHK(ensure(c, k1, std::max<uint64_t>(c->m, 1) * W * 8));
     if (any_fine)
@@ -3976,18 +4035,19 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     CHK(ensure(c, c->pair_h, c->x * 4));
     CHK(ensure(c, c->pair_b, c->x * 4));
     CHK(ensure(c, c->boff, (G + 1) * 4));
-    const uint32_t nbits = (uint32_t)__builtin_ctz(B);
+    CHK(ensure(c, c->rows, J ? (GR + 1) * 4 : 0));
+    const uint32_t nbits = nb + J;
     // 512 threads per 2048-k-mer tile (measured against 256 and 1024: the
     // staged form holds four tiles per CU, and 8 waves each hide more latency)
     constexpr int NT1 = 512;
     const bool stage1 = !(c->opts.flags & UC_FLAG_DIRECT_SCATTER) &&
-                        lmin_stage_bytes<W>(B, tile1, keep_src) <= c->lds_limit;
+                        lmin_stage_bytes<W>(R, tile1, keep_src) <= c->lds_limit;
 #define UC_S1(ST, C32)                                                                                              \
     do {                                                                                                           \
-        const size_t lds = ST ? lmin_stage_bytes<W>(B, tile1, keep_src) : lmin_lds_bytes(B, tile1 / 64);              \
+        const size_t lds = ST ? lmin_stage_bytes<W>(R, tile1, keep_src) : lmin_lds_bytes(R, tile1 / 64);              \
         CHK(allow_lds(c, k_lmin_scatter<W, IPT1 * BLOCK / NT1, ST, NT1, C32>, lds));                                \
         KLAUNCH(c, "k_lmin_scatter", (k_lmin_scatter<W, IPT1 * BLOCK / NT1, ST, NT1, C32>), (xcd_grid(T), NT1, lds), \
-                kin, P<BTile>(c->tiles), B, nbits, c->top_mask, c->bkt.p, P<uint32_t>(c->hist),                     \
+                kin, P<BTile>(c->tiles), R, nbits, c->top_mask, c->bkt.p, P<uint32_t>(c->hist),                     \
                 P<uint32_t>(c->xhist), P<uint64_t>(k1), any_fine ? nullptr : P<uint8_t>(c->flags),                  \
                 keep_src ? P<uint32_t>(s1) : nullptr, P<uint32_t>(c->pair_h), P<uint32_t>(c->pair_b),               \
                 any_fine ? P<uint16_t>(c->sub) : nullptr, tile_arg_xcd(T));                                         \
@@ -4000,10 +4060,12 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         else UC_S1(false, false);
     }
 #undef UC_S1
-    // the fine rows are the coarse rows when no set has a fine sort
+    // the fine rows are pass 1's rows when no second pass follows
     CHK(ensure(c, c->fboff, (F + 1) * 4));
-    KLAUNCH(c, "k_gather_boff", k_gather_boff, (grid_for(G + 1), BLOCK, 0), P<uint32_t>(c->hist),
-            sethb, setts, S, B, (uint32_t)c->m, mdev, P<uint32_t>(c->boff), any_fine ? nullptr : P<uint32_t>(c->fboff));
+    uint32_t *rows = J ? P<uint32_t>(c->rows) : P<uint32_t>(c->boff);
+    KLAUNCH(c, "k_gather_boff", k_gather_boff, (grid_for(GR + 1), BLOCK, 0), P<uint32_t>(c->hist), sethb, setts, S, R, J,
+            (uint32_t)c->m, mdev, row_first, rows, J ? P<uint32_t>(c->boff) : nullptr,
+            any_fine ? nullptr : P<uint32_t>(c->fboff));
     c->rows_valid = false;
     if (c->opts.flags & UC_FLAG_LOW_MEMORY) {
         // the codes, the input and the tile histogram are read by pass 1 and
@@ -4036,40 +4098,40 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         // for the direct two-word form (each measured best of 256/512/1024)
         constexpr int NT2 = W == 1 ? 512 : 1024;
         const bool stage2 = W == 1 && !(c->opts.flags & UC_FLAG_DIRECT_SCATTER) &&
-                            sub_lds_bytes<W>(round2, smax, keep_src, true, NT2 / 64) <= c->lds_limit;
+                            sub_lds_bytes<W>(round2, s1max, keep_src, true, NT2 / 64) <= c->lds_limit;
         c->tile2 = tile2;
-        // tiles: at most one partial tile per coarse bucket beyond m / tile2
-        const uint64_t T2 = G + (c->m + tile2 - 1) / tile2;
-        const uint64_t h2 = (uint64_t)smax * T2;  // histogram entries, upper bound
+        // tiles: at most one partial tile per row beyond m / tile2
+        const uint64_t T2 = GR + (c->m + tile2 - 1) / tile2;
+        const uint64_t h2 = (uint64_t)s1max * T2;  // histogram entries, upper bound
         CHK(ensure(c, c->tiles2, T2 * sizeof(BTile)));
         CHK(ensure(c, c->hist2, (h2 + 1) * 4));
-        CHK(ensure(c, c->cbhb, (G + 1) * 8));
-        CHK(ensure(c, c->cbts, (G + 1) * 4));
-        CHK(ensure(c, c->cbtf, (G + 1) * 4));
-        KLAUNCH(c, "k_plan2_prefix", k_plan2_prefix, (1, PLAN_NT, 0), P<uint32_t>(c->boff), P<uint32_t>(c->cbfirst),
-                (uint32_t)G, tile2, P<uint32_t>(c->cbts), P<uint32_t>(c->cbtf), P<uint64_t>(c->cbhb));
-        KLAUNCH(c, "k_plan2_tiles", k_plan2_tiles, (grid_for(T2), BLOCK, 0), P<uint32_t>(c->boff),
-                P<uint32_t>(c->cbfirst), P<uint32_t>(c->cbts), P<uint32_t>(c->cbtf), P<uint64_t>(c->cbhb), (uint32_t)G,
+        CHK(ensure(c, c->cbhb, (GR + 1) * 8));
+        CHK(ensure(c, c->cbts, (GR + 1) * 4));
+        CHK(ensure(c, c->cbtf, (GR + 1) * 4));
+        KLAUNCH(c, "k_plan2_prefix", k_plan2_prefix, (1, PLAN_NT, 0), rows, row_first,
+                (uint32_t)GR, tile2, P<uint32_t>(c->cbts), P<uint32_t>(c->cbtf), P<uint64_t>(c->cbhb));
+        KLAUNCH(c, "k_plan2_tiles", k_plan2_tiles, (grid_for(T2), BLOCK, 0), rows,
+                row_first, P<uint32_t>(c->cbts), P<uint32_t>(c->cbtf), P<uint64_t>(c->cbhb), (uint32_t)GR,
                 tile2, (uint32_t)T2, P<BTile>(c->tiles2));
-        KLAUNCH(c, "k_sub_count", k_sub_count, ((uint32_t)T2, SUB_COUNT_NT, smax * 4), P<uint16_t>(c->sub),
+        KLAUNCH(c, "k_sub_count", k_sub_count, ((uint32_t)T2, SUB_COUNT_NT, s1max * 4), P<uint16_t>(c->sub),
                 P<BTile>(c->tiles2), P<uint32_t>(c->hist2));
-        const uint32_t cpb = (smax + 63) / 64;  // column blocks per coarse bucket
+        const uint32_t cpb = (s1max + 63) / 64;  // column blocks per row
         CHK(ensure(c, c->colsum, F * 4 + 4));
-        KLAUNCH(c, "k_sub_colscan", k_sub_colscan, ((uint32_t)(G * cpb), BLOCK, 0), P<uint32_t>(c->hist2),
-                P<uint64_t>(c->cbhb), P<uint32_t>(c->cbts), P<uint32_t>(c->cbfirst), cpb, P<uint32_t>(c->colsum));
-        KLAUNCH(c, "k_sub_rows", k_sub_rows, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->colsum), P<uint32_t>(c->cbfirst),
-                P<uint32_t>(c->boff), (uint32_t)G, (uint32_t)c->m, mdev, P<uint32_t>(c->fboff));
+        KLAUNCH(c, "k_sub_colscan", k_sub_colscan, ((uint32_t)(GR * cpb), BLOCK, 0), P<uint32_t>(c->hist2),
+                P<uint64_t>(c->cbhb), P<uint32_t>(c->cbts), row_first, cpb, P<uint32_t>(c->colsum));
+        KLAUNCH(c, "k_sub_rows", k_sub_rows, ((uint32_t)GR, BLOCK, 0), P<uint32_t>(c->colsum), row_first,
+                rows, (uint32_t)GR, (uint32_t)c->m, mdev, P<uint32_t>(c->fboff));
         CHK(ensure(c, c->kmer, std::max<uint64_t>(c->m, 1) * W * 8));
         CHK(ensure(c, c->flags, c->m + 64));
         if (keep_src) CHK(ensure(c, c->src, c->m * 4));
         CHK(ensure(c, c->perm, c->m * 4));
 #define UC_S2(ST)                                                                                                   \
     do {                                                                                                           \
-        const size_t lds2 = sub_lds_bytes<W>(round2, smax, keep_src, ST, NT2 / 64);                                 \
+        const size_t lds2 = sub_lds_bytes<W>(round2, s1max, keep_src, ST, NT2 / 64);                                 \
         CHK(allow_lds(c, k_sub_scatter<W, ST, IPT2 * BLOCK / NT2, NT2>, lds2));                                    \
         KLAUNCH(c, "k_sub_scatter", (k_sub_scatter<W, ST, IPT2 * BLOCK / NT2, NT2>), (xcd_grid(T2), NT2, lds2),      \
                 P<BTile>(c->tiles2), P<uint16_t>(c->sub), P<uint32_t>(c->hist2), P<uint32_t>(c->fboff),             \
-                P<uint32_t>(c->cbfirst), P<uint64_t>(c->kmer2), keep_src ? P<uint32_t>(c->src2) : nullptr,          \
+                row_first, P<uint64_t>(c->kmer2), keep_src ? P<uint32_t>(c->src2) : nullptr,          \
                 P<uint64_t>(c->kmer), P<uint8_t>(c->flags), keep_src ? P<uint32_t>(c->src) : nullptr,               \
                 P<uint32_t>(c->perm), tile_arg_xcd(T2));                                                           \
     } while (0)

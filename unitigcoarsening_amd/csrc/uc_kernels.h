@@ -49,7 +49,7 @@ struct BTile {              // bucketing tile (one workgroup)
     uint32_t ts;            // tiles of the set / coarse bucket
     uint32_t tlocal;        // tile index inside it
     uint32_t fmask;         // pass 1: fine-bucket mask B*S-1 of the set; pass 2: S
-    uint32_t pad;
+    uint32_t split;         // pass 1: where the set's fine bits go (split_bits)
 };
 
 struct EGroup {             // edge-finding group: consecutive fine buckets of one
