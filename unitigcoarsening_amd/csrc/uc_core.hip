@@ -1970,8 +1970,31 @@ __global__ __launch_bounds__(1024) void k_edge_slice(const uint64_t *__restrict_
 // segments are ranked by pointer jumping over the sampled splitters only.
 // Emission then walks each segment again, copying its runs' characters.
 
-constexpr int CT_TILE = SCAN_TILE;  // slots per contraction tile
-static_assert(CT_TILE <= 2048, "a tile's list entries hold slot offsets in 11 bits");
+// LDS writes of one wave visible to the whole wave (no block barrier)
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Slots per contraction (and emission) tile: the fewest, from CT_MIN to
+// CT_MAX, whose tiles one scan workgroup takes, so that small jobs spread over
+// many workgroups and need no scan over several (a 10 k job in 2048-slot tiles
+// kept 5 of 256 CUs busy: k_head_emit 31 us).  A tile is one wave: nothing in
+// it waits at a barrier, and a CU's waves are in different phases (50 Mbp job,
+// emission: 512 slots and one wave 617 us, 1024 and two 603, 1024 and four 642,
+// 2048 and four 685, 2048 and eight 815; 45 M 63-mers 755, 782, 791, 798, 893).
+constexpr int CT_NT = 64;
+constexpr uint32_t CT_MIN = 64, CT_MAX = 512;
+static_assert(CT_MAX <= 2048, "a tile's list entries hold slot offsets in 11 bits");
+
+__host__ __device__ constexpr uint32_t ct_tile(uint64_t m)
+{
+    uint32_t t = CT_MIN;
+    while (t < CT_MAX && (m + t - 1) / t > (uint64_t)SCAN_TILE) t *= 2;
+    return t;
+}
 
 // the borrowed duplicate's out-edge moves to the home copy; the target keeps
 // its has-predecessor bit
@@ -2045,9 +2068,13 @@ __device__ __forceinline__ uint64_t mlist_entry(uint32_t off, bool multi, uint32
 // other heads add their count here and their length in k_chain_tail).
 // Segment records are kept where the chain kernels read them (segments that
 // end at or start from a sampled splitter); heads of several runs go to the
-// tile's list, written contiguously
-template <int NT>
-__global__ __launch_bounds__(NT) void k_seg_count(const uint64_t *__restrict__ rec, const uint32_t *__restrict__ hasp,
+// tile's list, written contiguously.  Most heads' unitigs are their first run;
+// the splitters that walk on (5% of the slots) are gathered first, so that one
+// thread takes one walk and all of a tile's chains of random reads are in
+// flight at once (with each thread walking its own slots one after another a
+// wave followed 2-3 walks at a time, eight times).
+template <int CT>
+__global__ __launch_bounds__(CT_NT) void k_seg_count(const uint64_t *__restrict__ rec, const uint32_t *__restrict__ hasp,
                                                      const uint8_t *__restrict__ flags, uint32_t m, uint32_t salt,
                                                      uint32_t shift, uint64_t *__restrict__ seg,
                                                      uint32_t *__restrict__ prevseg, uint32_t *__restrict__ list,
@@ -2055,11 +2082,11 @@ __global__ __launch_bounds__(NT) void k_seg_count(const uint64_t *__restrict__ r
                                                      uint32_t *__restrict__ cnt, uint64_t *__restrict__ tile_sum,
                                                      uint64_t *__restrict__ tile_cnt, uint32_t n_tiles)
 {
-    constexpr int ITEMS = CT_TILE / NT, NW = NT / 64;  // slots per thread; waves
-    __shared__ uint64_t red[NW];
+    constexpr int NT = CT_NT, ITEMS = CT / NT;  // slots per thread
+    __shared__ uint16_t walk[CT];  // slots that walk: heads of several runs, then sampled splitters
     const uint32_t ti = xcd_tile(n_tiles);
     if (ti == NONE) return;
-    const uint64_t base = (uint64_t)ti * CT_TILE;
+    const uint64_t base = (uint64_t)ti * CT;
     // flags and has-predecessor words of this thread's slots, all in flight
     // at once (the flag array has slack past its end, so no load is guarded)
     uint8_t f[ITEMS];
@@ -2070,9 +2097,9 @@ __global__ __launch_bounds__(NT) void k_seg_count(const uint64_t *__restrict__ r
         f[j] = s < m ? flags[s] : (uint8_t)F_BORROW;
         hw[j] = hasp[(s < m ? s : 0) >> 5];
     }
-    // splitters; sampled ones get list slots with one atomic per workgroup
+    // splitters; sampled ones get list slots with one atomic per tile
     bool hd[ITEMS], rd[ITEMS];
-    uint32_t nr = 0, nruns = 0;
+    uint32_t nr = 0, nruns = 0, nh = 0;
 #pragma unroll
     for (int j = 0; j < ITEMS; j++) {
         const uint32_t s = (uint32_t)(base + (uint64_t)j * NT + threadIdx.x);
@@ -2081,43 +2108,46 @@ __global__ __launch_bounds__(NT) void k_seg_count(const uint64_t *__restrict__ r
         rd[j] = cand && !hd[j] && sampled(s, salt, shift);
         nruns += cand;
         nr += rd[j];
+        nh += hd[j];
     }
-    // every splitter's first run record in flight at once
+    // every head's first run record in flight at once
     uint64_t first[ITEMS];
 #pragma unroll
-    for (int j = 0; j < ITEMS; j++)
-        first[j] = (hd[j] || rd[j]) ? rec[base + (uint64_t)j * NT + threadIdx.x] : 0ull;
+    for (int j = 0; j < ITEMS; j++) first[j] = hd[j] ? rec[base + (uint64_t)j * NT + threadIdx.x] : 0ull;
+    uint64_t acc = (uint64_t)nh << 32;
     uint32_t nm = 0;
 #pragma unroll
-    for (int j = 0; j < ITEMS; j++) nm += hd[j] && rec_next(first[j]) != NONE;
-    // one scan ranks both: sampled splitters (low half), list heads (high)
-    __shared__ uint64_t wtot[NW];
-    __shared__ uint32_t bbase;
-    const uint64_t both = ((uint64_t)nm << 32) | nr;
-    const uint64_t incl = wave_incl_scan(both);
-    const int w = threadIdx.x / 64;
-    if (__lane_id() == 63) wtot[w] = incl;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t t = 0;
-        for (int q = 0; q < NW; q++) t += wtot[q];
-        bbase = (uint32_t)t ? atomicAdd(cnt + C_LIST, (uint32_t)t) : 0u;
-        mcnt[ti] = (uint32_t)(t >> 32);
-    }
-    __syncthreads();
-    uint64_t pre = incl - both;
-    for (int q = 0; q < w; q++) pre += wtot[q];
-    uint32_t li = bbase + (uint32_t)pre;
-    uint64_t mi = base + (pre >> 32);
-    uint64_t acc = 0;
-    uint32_t nsplit = 0;
     for (int j = 0; j < ITEMS; j++) {
-        if (!(hd[j] || rd[j])) continue;
-        const uint32_t s = (uint32_t)(base + (uint64_t)j * NT + threadIdx.x);
-        nsplit++;
-        uint32_t r = rec_len(first[j]), v = rec_next(first[j]), steps = 1;
+        const bool on = hd[j] && rec_next(first[j]) != NONE;
+        if (hd[j] && !on) acc += rec_len(first[j]);
+        hd[j] = on;
+        nm += on;
+    }
+    // one scan ranks both: sampled splitters (low half), list heads (high)
+    const uint64_t both = ((uint64_t)nm << 32) | nr;
+    const uint64_t incl = wave_incl_scan(both), pre = incl - both, tot = __shfl(incl, 63, 64);
+    const uint32_t tm = (uint32_t)(tot >> 32), tr = (uint32_t)tot;
+    uint32_t bbase = 0;
+    if (threadIdx.x == 0) {
+        if (tr) bbase = atomicAdd(cnt + C_LIST, tr);
+        mcnt[ti] = tm;
+    }
+    bbase = __shfl(bbase, 0, 64);
+    uint32_t mi = (uint32_t)(pre >> 32), ri = tm + (uint32_t)pre;
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        if (hd[j]) walk[mi++] = (uint16_t)(j * NT + threadIdx.x);
+        if (rd[j]) walk[ri++] = (uint16_t)(j * NT + threadIdx.x);
+    }
+    wave_sync();
+    const uint32_t nsplit = nh + nr;
+    for (uint32_t i = threadIdx.x; i < tm + tr; i += NT) {
+        const bool head = i < tm;
+        const uint32_t off = walk[i], s = (uint32_t)base + off;
+        uint64_t rr = rec[s];
+        uint32_t r = rec_len(rr), v = rec_next(rr), steps = 1;
         while (v != NONE && !sampled(v, salt, shift)) {
-            const uint64_t rr = rec[v];
+            rr = rec[v];
             r += rec_len(rr);
             v = rec_next(rr);
             // in-degree <= 1 bounds every walk by m runs; the cap only guards
@@ -2128,19 +2158,23 @@ __global__ __launch_bounds__(NT) void k_seg_count(const uint64_t *__restrict__ r
                 break;
             }
         }
-        if (rd[j] || v != NONE) seg[s] = (uint64_t)r | ((uint64_t)v << 32);
-        if (hd[j] && rec_next(first[j]) != NONE) mlist[mi++] = mlist_entry(s - (uint32_t)base, v != NONE, r);
+        if (!head || v != NONE) seg[s] = (uint64_t)r | ((uint64_t)v << 32);
         if (v != NONE) prevseg[v] = s;
-        if (hd[j]) {
-            acc += 1ull << 32;
+        if (head) {
+            mlist[base + i] = mlist_entry(off, v != NONE, r);
             if (v == NONE) acc += r;
+        } else {
+            list[bbase + i - tm] = s;
         }
-        if (rd[j]) list[li++] = s;
     }
     // per-tile sums, no global atomics: (heads << 32 | head-segment lengths)
     // and (splitters << 32 | runs)
-    acc = block_reduce_n<uint64_t, NW>(acc, red);
-    const uint64_t sr = block_reduce_n<uint64_t, NW>(((uint64_t)nsplit << 32) | nruns, red);
+    uint64_t sr = ((uint64_t)nsplit << 32) | nruns;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        acc += __shfl_xor(acc, o, 64);
+        sr += __shfl_xor(sr, o, 64);
+    }
     if (threadIdx.x == 0) {
         tile_sum[ti] = acc;
         tile_cnt[ti] = sr;
@@ -2204,7 +2238,7 @@ __global__ void k_chain_round(const uint32_t *__restrict__ list, const uint32_t 
 __global__ void k_chain_tail(const uint32_t *__restrict__ list, const uint32_t *__restrict__ np,
                              const uint32_t *__restrict__ hasp, const uint64_t *__restrict__ chain,
                              const uint64_t *__restrict__ seg, uint32_t *__restrict__ ulen,
-                             uint64_t *__restrict__ tile_sum, uint32_t *__restrict__ nonconv)
+                             uint64_t *__restrict__ tile_sum, uint32_t ct, uint32_t *__restrict__ nonconv)
 {
     const uint32_t n = *np;
     bool bad = false;
@@ -2217,7 +2251,7 @@ __global__ void k_chain_tail(const uint32_t *__restrict__ list, const uint32_t *
         } else if ((uint32_t)(seg[r] >> 32) == NONE) {
             const uint32_t len = (uint32_t)(c >> 32) + (uint32_t)seg[r];
             ulen[a] = len;
-            atomicAdd((unsigned long long *)&tile_sum[a / CT_TILE], (unsigned long long)len);
+            atomicAdd((unsigned long long *)&tile_sum[a / ct], (unsigned long long)len);
         }
     }
     const uint64_t bal = __ballot(bad);
@@ -2333,14 +2367,6 @@ __device__ __forceinline__ uint32_t mlist_len(uint64_t e, const uint32_t *__rest
     return (e >> 11) & 1u ? ulen[t0 + (e & 0x7FFu)] : (uint32_t)(e >> 32);
 }
 
-// LDS writes of one wave visible to the whole wave (no block barrier)
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // four characters from four 2-bit codes (the low byte of b, first code in
 // the low bits), first character in the low byte
 __device__ __forceinline__ uint32_t chars4(uint32_t b)
@@ -2381,6 +2407,24 @@ __device__ __forceinline__ void put_kmer(char *o, uint64_t at, const Kmer<W> &x,
     for (; i < k; i++) o[i] = base_char(char_at<W>(x, i));
 }
 
+// the same at any LDS address: whole words (LDS takes them unaligned), the last
+// one over the end of the one before, so that every lane does the same k / 4
+// stores
+template <int W>
+__device__ __forceinline__ void put_kmer_lds(char *o, const Kmer<W> &x, uint32_t k)
+{
+    auto word = [&](uint32_t i) {
+        const uint32_t v = kmer_chars4<W>(x, i);
+        __builtin_memcpy(o + i, &v, 4);
+    };
+    uint32_t i = 0;
+    for (; i + 4 <= k; i += 4) word(i);
+    if (i < k && k >= 4)
+        word(k - 4);
+    else
+        for (; i < k; i++) o[i] = base_char(char_at<W>(x, i));
+}
+
 // byte i (0..15) of a 16-byte line
 __device__ __forceinline__ char line_byte(const uint4 &v, uint32_t i)
 {
@@ -2402,9 +2446,6 @@ __device__ __forceinline__ void copy_chars(char *o, const char *__restrict__ rch
     }
 }
 
-// one head's segment at o (address `at` modulo 4): first k-mer x, the later
-// characters of its run (record r), the characters of every later run up to
-// the next sampled splitter, '\n' when the unitig ends there
 // characters from .. len - 1 of the run with record r at slot s: from the
 // record when the run is short, else from rch
 __device__ __forceinline__ void put_run(char *o, uint64_t r, const char *__restrict__ rch, uint32_t s, uint32_t from,
@@ -2418,40 +2459,33 @@ __device__ __forceinline__ void put_run(char *o, uint64_t r, const char *__restr
     }
 }
 
-// a head's first run at o (address `at` modulo 4): its first k-mer x, the
-// later characters of its run (record r), '\n' when the run is the whole
-// unitig; the runs after it are written after every head's first run
-template <int W>
-__device__ __forceinline__ void put_first(char *o, uint64_t at, const Kmer<W> &x, uint64_t r,
-                                          const char *__restrict__ rch, uint32_t s, uint32_t k)
+// the part of a head's first run (record r) after its first k-mer, at o: its
+// later characters, '\n' when the run is the whole unitig; the runs after it
+// are written after every head's first run
+__device__ __forceinline__ void put_rest(char *o, uint64_t r, const char *__restrict__ rch, uint32_t s)
 {
-    put_kmer<W>(o, at, x, k);
     const uint32_t len = rec_len(r);
-    put_run(o + k, r, rch, s, 1, len);  // the head's own character is the k-th above
-    if (rec_next(r) == NONE) o[k + len - 1] = '\n';
+    put_run(o, r, rch, s, 1, len);  // the head's own character is its k-mer's last
+    if (rec_next(r) == NONE) o[len - 1] = '\n';
 }
 
-// LDS staging bytes per wave in k_head_emit (a range that does not fit is
-// written directly): 2 KiB for one-word k-mers, whose 256-thread groups
-// would lose residency with more (measured on MI355X: 2 KiB 0.95 ms, 3 KiB
-// 1.07 ms, unstaged 1.05 ms on the 50 Mbp job), 4 KiB for two-word k-mers
-// (2 KiB: 8.8 against 8.4 ms on the 300 Mbp instance)
+// LDS staging bytes per wave in k_head_emit: the text of 64 heads of short
+// unitigs, 64 (k + 2.4) bytes at 2.4 k-mers each (2.2 KB at k = 32, 4.3 KB at
+// k = 64); a range that does not fit is written directly
 template <int W>
-constexpr uint32_t emit_stage() { return W == 1 ? 2048 : 4096; }
+constexpr uint32_t emit_stage() { return W == 1 ? 2560 : 4608; }
 
-// LDS index of slot i of an emission tile (one pad word after every 8)
-__device__ __forceinline__ uint32_t tix(uint32_t i) { return i + (i >> 3); }
-
-// per tile: exclusive prefix of (1 << 32 | length) over heads -> text
-// offsets.  Every head writes its first run (put_first).  The 64 slots a
-// wave takes at a time own one contiguous text range; when the range fits
-// the wave's LDS stage, the heads write into LDS and the range goes out as
-// aligned 16-byte stores, else each head writes its bytes to HBM itself.  A
-// thread's next item (record and k-mer) is loaded while it writes the
+// Per tile: the live heads are gathered in slot order (39% of the slots:
+// walking the slots themselves left 61% of every wave's lanes idle through the
+// spelling, 0.85 ms on the 50 Mbp job), a scan of their lengths gives their
+// text offsets, and the wave takes 64 of them at a time: one contiguous text
+// range, spelled into its LDS stage (put_kmer_lds, put_rest) and
+// written as aligned 16-byte lines, or straight to HBM when it does not fit.
+// A thread's next head (record and k-mer) is loaded while it writes the
 // current one.  Then the heads of several runs (the tile's list) walk their
 // later runs up to the first sampled splitter, many walks in flight at once.
-template <int W, bool STAGE, int NT>
-__global__ __launch_bounds__(NT) void k_head_emit(const uint64_t *__restrict__ kmer, const uint64_t *__restrict__ rec,
+template <int W, int CT>
+__global__ __launch_bounds__(CT_NT) void k_head_emit(const uint64_t *__restrict__ kmer, const uint64_t *__restrict__ rec,
                                                      const char *__restrict__ rch, const uint32_t *__restrict__ hasp,
                                                      const uint8_t *__restrict__ flags,
                                                      const uint64_t *__restrict__ mlist, const uint32_t *__restrict__ mcnt,
@@ -2463,22 +2497,21 @@ __global__ __launch_bounds__(NT) void k_head_emit(const uint64_t *__restrict__ k
 {
     constexpr uint32_t STG = emit_stage<W>();
     if (gate && !pass_settled(gate, n_kmers)) return;  // (uniform over the grid)
-    constexpr int NW = NT / 64, CTI = CT_TILE / NT;  // waves; items per thread
-    // prefixes in slot order, then the tile's end; slot i at tix(i), one pad
-    // word after every 8, so that a thread's 8 consecutive slots (the scan
-    // below) sit 72 bytes from the next thread's: 4-way LDS bank access, as
-    // for any 64 lanes of 8-byte words, where 64 bytes put every lane on one
-    // of two bank pairs
-    __shared__ uint64_t tile[CT_TILE + CT_TILE / 8 + 1];
-    __shared__ uint64_t wsum[NW];
-    __shared__ __align__(16) char stage[STAGE ? NW : 1][STAGE ? STG : 16];
+    constexpr int NT = CT_NT, CTI = CT / NT;  // slots per thread
+    __shared__ uint64_t hmask[CTI];  // live heads of each 64 slots
+    __shared__ uint32_t gbase[CTI];  // heads before them in the tile
+    __shared__ __align__(16) uint32_t hpre[CT + 4];  // per head: its length, then the lengths before it
+    __shared__ uint16_t hslot[CT];   // per head: its slot in the tile
+    __shared__ uint32_t wsum[1];
+    __shared__ __align__(16) char stg[STG];
     const uint32_t ti = xcd_tile(n_tiles);
     if (ti == NONE) return;
-    const uint64_t t0 = (uint64_t)ti * CT_TILE;
-    uint32_t hd = 0;  // per item: live head
+    const uint64_t t0 = (uint64_t)ti * CT;
+    const uint32_t lane = threadIdx.x;
     // the tile's list of heads of several runs, its entries, and every
-    // item's flags, predecessor bit and run record, all in flight at once
+    // slot's flags, predecessor bit and run record, all in flight at once
     const uint32_t nml = mcnt[ti];
+    const uint64_t tb = tile_off[ti];
     uint32_t fh[CTI];
     uint64_t hr[CTI];
 #pragma unroll
@@ -2493,72 +2526,70 @@ __global__ __launch_bounds__(NT) void k_head_emit(const uint64_t *__restrict__ k
         const uint32_t e = (uint32_t)j * NT + threadIdx.x;
         ml[j] = e < nml ? mlist[t0 + e] : 0ull;
     }
-    // a live head (not borrowed, no predecessor) whose run is its unitig has
-    // its length now; the list fills in the others
+    // live heads (not borrowed, no predecessor), in slot order; a head whose
+    // run is its unitig has its length now, the list fills in the others
+    const uint64_t lt = (1ull << lane) - 1ull;
+    uint32_t nh = 0;
 #pragma unroll
     for (int j = 0; j < CTI; j++) {
-        uint64_t v = 0;
-        if (!(fh[j] & (F_BORROW | 0x100u))) {
-            hd |= 1u << j;
-            if (rec_next(hr[j]) == NONE) v = (1ull << 32) | rec_len(hr[j]);
+        const bool h = !(fh[j] & (F_BORROW | 0x100u));
+        const uint64_t mask = __ballot(h);
+        if (lane == 0) {
+            hmask[j] = mask;
+            gbase[j] = nh;
         }
-        tile[tix(j * NT + threadIdx.x)] = v;
+        if (h) {
+            const uint32_t i = nh + (uint32_t)__popcll(mask & lt);
+            hslot[i] = (uint16_t)(j * NT + lane);
+            hpre[i] = rec_next(hr[j]) == NONE ? rec_len(hr[j]) : 0u;
+        }
+        nh += (uint32_t)__popcll(mask);
     }
-    __syncthreads();
+    wave_sync();
+    auto head_of = [&](uint32_t slot) {  // index of the head at a slot of the tile
+        return gbase[slot >> 6] + (uint32_t)__popcll(hmask[slot >> 6] & ((1ull << (slot & 63)) - 1ull));
+    };
 #pragma unroll
     for (int j = 0; j < CTI; j++) {
         const uint32_t e = (uint32_t)j * NT + threadIdx.x;
-        if (e < nml) tile[tix(ml[j] & 0x7FFu)] = (1ull << 32) | mlist_len(ml[j], ulen, t0);
+        if (e < nml) hpre[head_of((uint32_t)(ml[j] & 0x7FFu))] = mlist_len(ml[j], ulen, t0);
     }
-    __syncthreads();
-    uint64_t loc[CTI];
-    uint64_t run = 0;
-#pragma unroll
-    for (int j = 0; j < CTI; j++) {
-        loc[j] = run;
-        run += tile[tix(threadIdx.x * CTI + j)];
-    }
-    const uint64_t incl = wave_incl_scan(run);
-    const int w = threadIdx.x / 64;
-    if (__lane_id() == 63) wsum[w] = incl;
-    __syncthreads();
-    uint64_t wpre = 0;
-    for (int i = 0; i < w; i++) wpre += wsum[i];
-    const uint64_t excl = tile_off[ti] + wpre + incl - run;
-#pragma unroll
-    for (int j = 0; j < CTI; j++) tile[tix(threadIdx.x * CTI + j)] = excl + loc[j];
-    if (threadIdx.x == NT - 1) tile[tix(CT_TILE)] = excl + run;
-    __syncthreads();
-    char *stg = stage[STAGE ? w : 0];
-    const uint32_t lane = __lane_id();
-    const uint32_t s0 = (uint32_t)t0 + threadIdx.x;
+    wave_sync();
+    const uint32_t all = block_excl_scan_n<NT>(hpre, nh, wsum);
+    if (lane == 0) hpre[nh] = all;
+    wave_sync();
+    // text offset of head i (and the end of the last one at i = nh)
+    const uint64_t tbase = (tb & 0xFFFFFFFFull) + (tb >> 32) * k;
+    auto offset = [&](uint32_t i) { return tbase + hpre[i] + (uint64_t)i * k; };
     Kmer<W> nx{};
     uint64_t nr = 0;
-    if (hd & 1u) {
-        nx = load_kmer<W>(kmer, s0, ~0ull);
-        nr = rec[s0];
-    }
+    uint32_t ns = 0;
+    auto load = [&](uint32_t i) {
+        if (i < nh) {
+            ns = (uint32_t)t0 + hslot[i];
+            nx = load_kmer<W>(kmer, ns, ~0ull);
+            nr = rec[ns];
+        }
+    };
+    load(lane);
 #pragma unroll 1
-    for (uint32_t j = 0; j < (uint32_t)CTI; j++) {
-        const uint32_t s = s0 + j * NT;
+    for (uint32_t i0 = 0; i0 < nh; i0 += NT) {  // uniform over the wave
+        const uint32_t i = i0 + lane, s = ns;
         const uint64_t r = nr;
         const Kmer<W> x = nx;
-        if ((hd >> (j + 1)) & 1u) {
-            nx = load_kmer<W>(kmer, s + NT, ~0ull);
-            nr = rec[s + NT];
-        }
-        const bool h = (hd >> j) & 1u;
-        const uint64_t pre = tile[tix(j * NT + threadIdx.x)];
-        const uint64_t off = (pre & 0xFFFFFFFFull) + (pre >> 32) * k;
-        // the wave's text range [r0, r1): from its first slot to the slot after its last
-        const uint32_t li = j * NT + (uint32_t)w * 64;
-        const uint64_t p0 = tile[tix(li)], p1 = tile[tix(li + 64)];
-        const uint64_t r0 = (p0 & 0xFFFFFFFFull) + (p0 >> 32) * k, r1 = (p1 & 0xFFFFFFFFull) + (p1 >> 32) * k;
+        load(i + NT);
+        const bool h = i < nh;
+        // the wave's text range [r0, r1)
+        const uint64_t r0 = offset(i0), r1 = offset(i0 + 64 < nh ? i0 + 64 : nh);
+        const uint64_t off = h ? offset(i) : 0;
         const uint64_t a = r0 & ~15ull;  // staged from r0's 16-byte line
-        if (STAGE && r1 - a <= STG) {  // uniform over the wave
-            // (the bytes of runs after a head's first run are written by later
-            // kernels over what the stage holds there)
-            if (h) put_first<W>(stg + (off - a), off, x, r, rch, s, k);
+        if (r1 - a <= STG) {             // uniform over the wave
+            // (the bytes of runs after a head's first run are written later
+            // over what the stage holds there)
+            if (h) {
+                put_kmer_lds<W>(stg + (off - a), x, k);
+                put_rest(stg + (off - a) + k, r, rch, s);
+            }
             wave_sync();
             // whole lines [f, e) as 16-byte stores; the partial first and last
             // lines byte by byte, one lane per byte
@@ -2570,12 +2601,13 @@ __global__ __launch_bounds__(NT) void k_head_emit(const uint64_t *__restrict__ k
             if (lane < 32 && hb < hlim && (lane < 16 || e >= f)) text[hb] = stg[hb - a];
             wave_sync();
         } else if (h) {
-            put_first<W>(text + off, off, x, r, rch, s, k);
+            put_kmer<W>(text + off, off, x, k);
+            put_rest(text + off + k, r, rch, s);
         }
     }
     // the later runs of the heads of several runs (the tile's list), over
-    // what the waves' stores above left there: the whole tile's text range
-    // belongs to this group, so one barrier orders the two
+    // what the stores above left there (the whole tile's text range belongs
+    // to this wave, and its stores to one address keep their order)
     __syncthreads();
 #pragma unroll 1
     for (int j = 0; j < CTI; j++) {
@@ -2583,8 +2615,7 @@ __global__ __launch_bounds__(NT) void k_head_emit(const uint64_t *__restrict__ k
         if (e >= nml) break;
         const uint32_t ls = (uint32_t)(ml[j] & 0x7FFu);
         const uint32_t s = (uint32_t)t0 + ls;
-        const uint64_t pre = tile[tix(ls)];
-        const uint64_t off = (pre & 0xFFFFFFFFull) + (pre >> 32) * k;
+        const uint64_t off = offset(head_of(ls));
         uint64_t r = rec[s];
         uint64_t p = off + k + rec_len(r) - 1;
         uint32_t v = rec_next(r), steps = 0;
@@ -2645,7 +2676,7 @@ __global__ __launch_bounds__(BLOCK) void k_set_offsets(const uint32_t *__restric
                                                        const uint64_t *__restrict__ mlist,
                                                        const uint32_t *__restrict__ mcnt,
                                                        const uint32_t *__restrict__ ulen,
-                                                       const uint64_t *__restrict__ tile_off, uint32_t m,
+                                                       const uint64_t *__restrict__ tile_off, uint32_t m, uint32_t ct,
                                                        const uint64_t *__restrict__ total, uint64_t *__restrict__ out,
                                                        const uint32_t *__restrict__ gate, uint32_t n_kmers)
 {
@@ -2657,8 +2688,8 @@ __global__ __launch_bounds__(BLOCK) void k_set_offsets(const uint32_t *__restric
         if (threadIdx.x == 0) out[s] = *total;  // (unitigs << 32 | k-mers) of the whole job
         return;
     }
-    const uint32_t t = sb / CT_TILE;
-    const uint64_t t0 = (uint64_t)t * CT_TILE;
+    const uint32_t t = sb / ct;
+    const uint64_t t0 = (uint64_t)t * ct;
     uint64_t acc = 0;
     for (uint32_t x = (uint32_t)t0 + threadIdx.x; x < sb; x += BLOCK)
         if (live_head(flags, hasp, x)) {
@@ -4555,12 +4586,25 @@ void drop_pass_graph(uc_ctx *c)
     c->cgraph_key.clear();
 }
 
+// f with the contraction tile as a constant
+template <typename F>
+int with_ct(uint32_t ct, F f)
+{
+    switch (ct) {
+    case 64: return f(std::integral_constant<int, 64>{});
+    case 128: return f(std::integral_constant<int, 128>{});
+    case 256: return f(std::integral_constant<int, 256>{});
+    default: return f(std::integral_constant<int, 512>{});
+    }
+}
+
 // With `defer`, the speculative pass is only launched: its counters stay on
 // the device for finish_deferred().
 int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true, bool defer = false)
 {
     const uint32_t m = (uint32_t)c->m;
-    const uint64_t T = (c->m + CT_TILE - 1) / CT_TILE;
+    const uint32_t ct = ct_tile(c->m);
+    const uint64_t T = (c->m + ct - 1) / ct;
     uint32_t *cnt = P<uint32_t>(c->small);
     const uint32_t *np = cnt + C_LIST;
     uint64_t *ca = P<uint64_t>(c->chainA), *cb = P<uint64_t>(c->chainB);
@@ -4568,13 +4612,13 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
     // unitig-length scan; everything up to the counter read
     auto walks = [&]() -> int {
         CHK(fill<uint32_t>(c, cnt, C_SLICE, 0u));  // (the edge phase's slice flag stays)
-        // 256 threads, 8 slots each: the walks of a thread's splitters
-        // overlap (measured on MI355X, 50 Mbp job: 0.30 ms; 128 threads
-        // 0.35, 512 threads 0.37, 1024 threads 0.74)
-        KLAUNCH(c, "k_seg_count", k_seg_count<256>, (xcd_grid(T), 256, 0), P<uint64_t>(c->rec), P<uint32_t>(c->hasp),
-                P<uint8_t>(c->flags), m, c->salt, c->shift, P<uint64_t>(c->seg), P<uint32_t>(c->prevseg),
-                P<uint32_t>(c->list), P<uint64_t>(c->mlist), P<uint32_t>(c->mcnt), cnt, P<uint64_t>(c->tsum),
-                P<uint64_t>(c->tcnt), tile_arg(c, T));
+        CHK(with_ct(ct, [&](auto CT) -> int {
+            KLAUNCH(c, "k_seg_count", k_seg_count<CT.value>, (xcd_grid(T), CT_NT, 0), P<uint64_t>(c->rec),
+                    P<uint32_t>(c->hasp), P<uint8_t>(c->flags), m, c->salt, c->shift, P<uint64_t>(c->seg),
+                    P<uint32_t>(c->prevseg), P<uint32_t>(c->list), P<uint64_t>(c->mlist), P<uint32_t>(c->mcnt), cnt,
+                    P<uint64_t>(c->tsum), P<uint64_t>(c->tcnt), tile_arg(c, T));
+            return UC_OK;
+        }));
         CHK(scan_excl<uint64_t>(c, P<uint64_t>(c->tcnt), P<uint64_t>(c->tcnt), T,
                                 reinterpret_cast<uint64_t *>(cnt + C_TOT), c->scan_tmp));
         return UC_OK;
@@ -4595,7 +4639,7 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
             std::swap(a, b);
         }
         KLAUNCH(c, "k_chain_tail", k_chain_tail, (g, BLOCK, 0), P<uint32_t>(c->list), np, P<uint32_t>(c->hasp), a,
-                P<uint64_t>(c->seg), P<uint32_t>(c->ulen), P<uint64_t>(c->tsum), cnt + C_NONCONV);
+                P<uint64_t>(c->seg), P<uint32_t>(c->ulen), P<uint64_t>(c->tsum), ct, cnt + C_NONCONV);
         return totals();
     };
     uint32_t h[C_WORDS];
@@ -4663,7 +4707,7 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
             }
             KLAUNCH(c, "k_chain_tail", k_chain_tail, (g, BLOCK, 0), P<uint32_t>(c->list), np,
                     P<uint32_t>(c->hasp), ca, P<uint64_t>(c->seg), P<uint32_t>(c->ulen), P<uint64_t>(c->tsum),
-                    cnt + C_NONCONV);
+                    ct, cnt + C_NONCONV);
         }
         CHK(totals());
     }
@@ -4738,7 +4782,7 @@ int cut_cycles(uc_ctx *c, uint64_t *n_cut)
 // every array a contraction pass writes or reads besides the edge result
 int ensure_contraction(uc_ctx *c)
 {
-    const uint64_t T = (c->m + CT_TILE - 1) / CT_TILE;
+    const uint64_t T = (c->m + ct_tile(c->m) - 1) / ct_tile(c->m);
     CHK(ensure(c, c->small, C_WORDS * 4));
     CHK(ensure(c, c->tcnt, (T + 1) * 8));
     CHK(ensure(c, c->seg, c->m * 8));
@@ -4847,7 +4891,8 @@ template <int W>
 int run_emit(uc_ctx *c)
 {
     const uint32_t m = (uint32_t)c->m;
-    const uint64_t T = (c->m + CT_TILE - 1) / CT_TILE;
+    const uint32_t ct = ct_tile(c->m);
+    const uint64_t T = (c->m + ct - 1) / ct;
     if (c->text_fixed) {
         // the caller's buffer (uc_compact_noalloc); the kernels write bytes [0, text_bytes) only
         if (c->text.cap < c->text_bytes)
@@ -4875,14 +4920,13 @@ int run_emit(uc_ctx *c)
     // a pass the host has not checked: the kernels check it themselves
     const uint32_t *gate = c->deferred ? cnt : nullptr;
     if (m) {
-        // one-word k-mers from 256-thread groups, wider ones from 512-thread
-        // groups, both staged in LDS (each measured faster than the other
-        // choices on MI355X)
-        constexpr int NT = W == 1 ? 256 : 512;
-        KLAUNCH(c, "k_head_emit", (k_head_emit<W, true, NT>), (xcd_grid(T), NT, 0), P<uint64_t>(c->kmer),
-                P<uint64_t>(c->rec), P<char>(c->rch), P<uint32_t>(c->hasp), P<uint8_t>(c->flags),
-                P<uint64_t>(c->mlist), P<uint32_t>(c->mcnt), P<uint32_t>(c->ulen), P<uint64_t>(c->tsum), m, c->k,
-                c->salt, c->shift, htoff, P<char>(c->text), tile_arg(c, T), gate, (uint32_t)c->n);
+        CHK(with_ct(ct, [&](auto CT) -> int {
+            KLAUNCH(c, "k_head_emit", (k_head_emit<W, CT.value>), (xcd_grid(T), CT_NT, 0), P<uint64_t>(c->kmer),
+                    P<uint64_t>(c->rec), P<char>(c->rch), P<uint32_t>(c->hasp), P<uint8_t>(c->flags),
+                    P<uint64_t>(c->mlist), P<uint32_t>(c->mcnt), P<uint32_t>(c->ulen), P<uint64_t>(c->tsum), m, c->k,
+                    c->salt, c->shift, htoff, P<char>(c->text), tile_arg(c, T), gate, (uint32_t)c->n);
+            return UC_OK;
+        }));
     }
     if (c->deferred || c->n_list) {
         // (the list's length is read by the kernel: a deferred pass has not
@@ -4898,7 +4942,7 @@ int run_emit(uc_ctx *c)
         CHK(ensure(c, c->setoff, (c->n_sets + 1) * 8));
         KLAUNCH(c, "k_set_offsets", k_set_offsets, (c->n_sets + 1, BLOCK, 0), P<uint32_t>(c->boff), c->n_sets,
                 c->B, P<uint32_t>(c->hasp), P<uint8_t>(c->flags), P<uint64_t>(c->rec), P<uint64_t>(c->mlist),
-                P<uint32_t>(c->mcnt), P<uint32_t>(c->ulen), P<uint64_t>(c->tsum), m,
+                P<uint32_t>(c->mcnt), P<uint32_t>(c->ulen), P<uint64_t>(c->tsum), m, ct,
                 reinterpret_cast<const uint64_t *>(cnt + C_TOT + 2), P<uint64_t>(c->setoff), gate, (uint32_t)c->n);
     }
     return c->deferred ? finish_deferred(c) : set_ranges(c);
