@@ -356,11 +356,28 @@ __device__ __forceinline__ T block_reduce(T v, T *sh)
     return block_reduce_n<T, WAVES>(v, sh);
 }
 
+// One or two scans in a launch (the bucketing scans its tile histogram and its
+// crossing counts at once): workgroups below a.nb take a's tiles, the rest b's.
 template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_scan_reduce(const T *__restrict__ in, uint64_t n, T *__restrict__ partial)
+struct ScanArgs {
+    const T *in;
+    T *out;
+    uint64_t n;
+    uint32_t nb;    // tiles
+    T *partial;     // tile sums (nb > 1)
+    T *total;       // the sum, when given, and a copy of it
+    T *total2;
+};
+
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_scan_reduce(ScanArgs<T> a, ScanArgs<T> b)
 {
     __shared__ T sh[WAVES];
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
+    const bool second = blockIdx.x >= a.nb;
+    const T *__restrict__ in = second ? b.in : a.in;
+    const uint64_t n = second ? b.n : a.n;
+    const uint32_t bl = second ? blockIdx.x - a.nb : blockIdx.x;
+    const uint64_t base = (uint64_t)bl * SCAN_TILE;
     T s = 0;
 #pragma unroll
     for (int j = 0; j < SCAN_ITEMS; j++) {
@@ -368,23 +385,39 @@ __global__ __launch_bounds__(BLOCK) void k_scan_reduce(const T *__restrict__ in,
         if (i < n) s += in[i];
     }
     s = block_reduce(s, sh);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
+    if (threadIdx.x == 0) (second ? b.partial : a.partial)[bl] = s;
 }
 
-// exclusive scan of one tile per block; `offset` holds per-block exclusive
-// offsets (or is null); the block owning the last element writes the total
-// (and a copy of it at `total2`, when given)
-template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_scan_tile(const T *in, T *out, uint64_t n, const T *__restrict__ offset,
-                                                     T *__restrict__ total, T *__restrict__ total2)
+// exclusive scan of one tile per workgroup.  A tile's offset is the sum of the
+// tile sums before it, which every workgroup adds up itself (SUMS: a scan of
+// the sums in a launch of its own costs more up to SCAN_FLAT of them), or its
+// entry of the scanned sums.  The workgroup owning the last element writes the
+// total.
+template <typename T, bool SUMS>
+__global__ __launch_bounds__(BLOCK) void k_scan_tile(ScanArgs<T> a, ScanArgs<T> b)
 {
     __shared__ T tile[SCAN_TILE];
     __shared__ T wsum[WAVES];
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
+    const bool second = blockIdx.x >= a.nb;
+    const T *in = second ? b.in : a.in;
+    T *out = second ? b.out : a.out;
+    const T *__restrict__ partial = second ? b.partial : a.partial;
+    const uint64_t n = second ? b.n : a.n;
+    const uint32_t bl = second ? blockIdx.x - a.nb : blockIdx.x, nb = second ? b.nb : a.nb;
+    const uint64_t base = (uint64_t)bl * SCAN_TILE;
 #pragma unroll
     for (int j = 0; j < SCAN_ITEMS; j++) {
         uint64_t i = base + (uint64_t)j * BLOCK + threadIdx.x;
         tile[j * BLOCK + threadIdx.x] = i < n ? in[i] : T(0);
+    }
+    T boff = 0;
+    if (nb > 1) {
+        if constexpr (SUMS) {
+            for (uint32_t i = threadIdx.x; i < bl; i += BLOCK) boff += partial[i];
+            boff = block_reduce(boff, wsum);
+        } else {
+            boff = partial[bl];
+        }
     }
     __syncthreads();
     T loc[SCAN_ITEMS];
@@ -403,7 +436,6 @@ __global__ __launch_bounds__(BLOCK) void k_scan_tile(const T *in, T *out, uint64
         if (i < w) wpre += wsum[i];
         btot += wsum[i];
     }
-    const T boff = offset ? offset[blockIdx.x] : T(0);
     const T excl = boff + wpre + incl - run;
 #pragma unroll
     for (int j = 0; j < SCAN_ITEMS; j++) tile[threadIdx.x * SCAN_ITEMS + j] = excl + loc[j];
@@ -414,6 +446,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_tile(const T *in, T *out, uint64
         if (i < n) out[i] = tile[j * BLOCK + threadIdx.x];
     }
     if (threadIdx.x == 0 && base + SCAN_TILE >= n) {
+        T *total = second ? b.total : a.total, *total2 = second ? b.total2 : a.total2;
         if (total) *total = boff + btot;
         if (total2) *total2 = boff + btot;
     }
@@ -1588,6 +1621,46 @@ __global__ __launch_bounds__(BLOCK) void k_plan_write(const uint32_t *__restrict
     if (ng) pack_groups(fboff, f0, v0, v1, gmax, groups + base, nullptr, nullptr);
 }
 
+// The whole plan of a small job of one set in one workgroup, a thread per run
+// of fine buckets (the three launches of the general form and the fill before
+// them take 15 us on a 10 k job).  gfirst[G + 1] gets the oversized count,
+// gfirst[G + 2 ..] a copy of two counters (tot, when given).
+constexpr int PLAN_ONE_NT = 1024;
+
+__global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__restrict__ fboff, uint32_t G, uint32_t S,
+                                                          uint32_t gmax, uint32_t *__restrict__ gfirst,
+                                                          EGroup *__restrict__ groups, uint32_t *__restrict__ over,
+                                                          const uint32_t *__restrict__ tot)
+{
+    __shared__ uint32_t wsum[PLAN_ONE_NT / 64];
+    __shared__ uint32_t n_over;
+    if (threadIdx.x == 0) n_over = 0;
+    __syncthreads();
+    const uint32_t rp = (S + PLAN_RUN - 1) / PLAN_RUN;  // runs per coarse bucket
+    const uint32_t g = threadIdx.x / rp, j = threadIdx.x % rp;
+    const uint32_t v0 = j * PLAN_RUN, v1 = min(S, v0 + PLAN_RUN);
+    const uint32_t ng = g < G ? pack_groups(fboff, g * S, v0, v1, gmax, nullptr, over, &n_over) : 0u;
+    const uint32_t incl = wave_incl_scan(ng);
+    const int w = threadIdx.x / 64;
+    if (__lane_id() == 63) wsum[w] = incl;
+    __syncthreads();
+    uint32_t base = incl - ng, all = 0;
+    for (int q = 0; q < PLAN_ONE_NT / 64; q++) {
+        if (q < w) base += wsum[q];
+        all += wsum[q];
+    }
+    if (g < G && j == 0) gfirst[g] = base;
+    if (ng) pack_groups(fboff, g * S, v0, v1, gmax, groups + base, nullptr, nullptr);
+    if (threadIdx.x == 0) {
+        gfirst[G] = all;
+        gfirst[G + 1] = n_over;
+        if (tot) {
+            gfirst[G + 2] = tot[0];
+            gfirst[G + 3] = tot[1];
+        }
+    }
+}
+
 // ---- the LDS form: one workgroup stages a group of consecutive fine buckets
 // (k-mers) in LDS and runs insert, lookup and resolve against an LDS table;
 // each thread keeps its own slots' flags and last characters in registers.
@@ -2256,6 +2329,103 @@ __global__ void k_chain_tail(const uint32_t *__restrict__ list, const uint32_t *
     }
     const uint64_t bal = __ballot(bad);
     if (__lane_id() == 0 && bal) atomicAdd(nonconv, (uint32_t)__popcll(bal));
+}
+
+// Chain ranking, unitig lengths and the totals of a small job in one workgroup
+// (the same steps as k_chain_init, SPEC_ROUNDS of k_chain_round, k_chain_tail
+// and the scans of the tile sums, which are four to ten launches of 3-5 us
+// each with next to nothing in them): up to CHAIN_ONE_TILES tiles, and as many
+// sampled splitters as its threads can stride over.
+constexpr int CHAIN_ONE_NT = 1024;
+constexpr uint32_t CHAIN_ONE_TILES = 6144, CHAIN_ONE_LIST = 16384;
+
+__global__ __launch_bounds__(CHAIN_ONE_NT) void k_chain_one(const uint32_t *__restrict__ list, uint32_t *cnt,
+                                                            const uint32_t *__restrict__ hasp,
+                                                            const uint32_t *__restrict__ prevseg,
+                                                            const uint64_t *__restrict__ seg, uint64_t *chainA,
+                                                            uint64_t *chainB, uint32_t *__restrict__ ulen,
+                                                            uint64_t *__restrict__ tile_sum,
+                                                            const uint64_t *__restrict__ tile_cnt, uint32_t T, uint32_t ct)
+{
+    constexpr int NW = CHAIN_ONE_NT / 64;
+    extern __shared__ uint64_t sums[];  // T
+    __shared__ uint64_t wtot[NW];
+    __shared__ uint32_t red[NW];
+    uint64_t splits = 0;
+    for (uint32_t i = threadIdx.x; i < T; i += CHAIN_ONE_NT) {
+        sums[i] = tile_sum[i];
+        splits += tile_cnt[i];
+    }
+    const uint32_t n = cnt[C_LIST];
+    for (uint32_t i = threadIdx.x; i < n; i += CHAIN_ONE_NT) {
+        const uint32_t r = list[i], a = prevseg[r];
+        chainA[r] = (uint64_t)a | ((uint64_t)(uint32_t)seg[a] << 32);
+    }
+    uint64_t *cin = chainA, *cout = chainB;
+    for (uint32_t round = 0; round < SPEC_ROUNDS; round++) {
+        // (the barrier orders the entries that other waves of this workgroup
+        // wrote; fences for the whole device took 10 us more)
+        __syncthreads();
+        uint32_t act = 0;
+        for (uint32_t i = threadIdx.x; i < n; i += CHAIN_ONE_NT) {
+            const uint32_t r = list[i];
+            const uint64_t c = cin[r];
+            const uint32_t a = (uint32_t)c;
+            if (!has_pred(hasp, a)) {
+                cout[r] = c;
+            } else {
+                const uint64_t c2 = cin[a];
+                const uint32_t a2 = (uint32_t)c2;
+                cout[r] = (uint64_t)a2 | ((uint64_t)((uint32_t)(c >> 32) + (uint32_t)(c2 >> 32)) << 32);
+                act += has_pred(hasp, a2);
+            }
+        }
+        act = block_reduce_n<uint32_t, NW>(act, red);
+        if (threadIdx.x == 0) cnt[C_ACTIVE + round] = act;
+        uint64_t *t = cin;
+        cin = cout;
+        cout = t;
+    }
+    __syncthreads();
+    uint32_t bad = 0;
+    for (uint32_t i = threadIdx.x; i < n; i += CHAIN_ONE_NT) {
+        const uint32_t r = list[i];
+        const uint64_t c = cin[r], sg = seg[r];
+        const uint32_t a = (uint32_t)c;
+        if (has_pred(hasp, a)) {
+            bad++;  // no head behind this chain: an isolated cycle
+        } else if ((uint32_t)(sg >> 32) == NONE) {
+            const uint32_t len = (uint32_t)(c >> 32) + (uint32_t)sg;
+            ulen[a] = len;
+            atomicAdd((unsigned long long *)&sums[a / ct], (unsigned long long)len);
+        }
+    }
+    bad = block_reduce_n<uint32_t, NW>(bad, red);
+    splits = block_reduce_n<uint64_t, NW>(splits, wtot);
+    // exclusive scan of the tile sums, a stretch of them per thread
+    const uint32_t per = (T + CHAIN_ONE_NT - 1) / CHAIN_ONE_NT;
+    const uint32_t b0 = min(T, threadIdx.x * per), b1 = min(T, b0 + per);
+    uint64_t loc = 0;
+    for (uint32_t i = b0; i < b1; i++) loc += sums[i];
+    const uint64_t incl = wave_incl_scan(loc);
+    const int w = threadIdx.x / 64;
+    if (__lane_id() == 63) wtot[w] = incl;
+    __syncthreads();
+    uint64_t pre = incl - loc, tot = 0;
+    for (int q = 0; q < NW; q++) {
+        if (q < w) pre += wtot[q];
+        tot += wtot[q];
+    }
+    for (uint32_t i = b0; i < b1; i++) {
+        const uint64_t v = sums[i];
+        tile_sum[i] = pre;
+        pre += v;
+    }
+    if (threadIdx.x == 0) {
+        cnt[C_NONCONV] = bad;
+        *reinterpret_cast<uint64_t *>(cnt + C_TOT) = splits;
+        *reinterpret_cast<uint64_t *>(cnt + C_TOT + 2) = tot;
+    }
 }
 
 // ---- isolated cycles (only when some k-mers are not reached from a head) --
@@ -3329,8 +3499,8 @@ int allow_lds(uc_ctx *c, K kernel, size_t bytes)
     return UC_OK;
 }
 
-// exclusive scan of n values (in == out allowed); *d_total gets the sum.
-// Block sums of every recursion level live in `tmp`.
+// scratch of an exclusive scan of n values (in == out allowed): the tile sums
+// of every level
 template <typename T>
 size_t scan_scratch(uint64_t n)
 {
@@ -3340,20 +3510,35 @@ size_t scan_scratch(uint64_t n)
     return bytes;
 }
 
+constexpr uint64_t SCAN_FLAT = 4096;  // tile sums a workgroup adds up itself
+
 template <typename T>
-int scan_level(uc_ctx *c, const T *in, T *out, uint64_t n, T *d_total, T *d_total2, char *tmp)
+int scan_pair(uc_ctx *c, ScanArgs<T> a, ScanArgs<T> b, char *tmp)
 {
-    const uint64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-    if (nb <= 1) {
-        KLAUNCH(c, "k_scan_tile", k_scan_tile<T>, (1, BLOCK, 0), in, out, n, nullptr, d_total, d_total2);
+    const uint64_t most = std::max(a.nb, b.nb);
+    char *next = tmp;
+    for (ScanArgs<T> *x : {&a, &b}) {
+        x->partial = reinterpret_cast<T *>(next);
+        if (x->nb > 1) next += ((x->nb + 1) * sizeof(T) + 255) / 256 * 256;
+    }
+    if (most > 1) KLAUNCH(c, "k_scan_reduce", k_scan_reduce<T>, (a.nb + b.nb, BLOCK, 0), a, b);
+    if (most <= SCAN_FLAT) {
+        KLAUNCH(c, "k_scan_tile", (k_scan_tile<T, true>), (a.nb + b.nb, BLOCK, 0), a, b);
         return UC_OK;
     }
-    T *partial = reinterpret_cast<T *>(tmp);
-    char *next = tmp + ((nb + 1) * sizeof(T) + 255) / 256 * 256;
-    KLAUNCH(c, "k_scan_reduce", k_scan_reduce<T>, ((uint32_t)nb, BLOCK, 0), in, n, partial);
-    CHK(scan_level<T>(c, partial, partial, nb, nullptr, nullptr, next));
-    KLAUNCH(c, "k_scan_tile", k_scan_tile<T>, ((uint32_t)nb, BLOCK, 0), in, out, n, partial, d_total, d_total2);
+    for (const ScanArgs<T> &x : {a, b}) {
+        if (x.nb <= 1) continue;
+        ScanArgs<T> up{x.partial, x.partial, x.nb, (uint32_t)((x.nb + SCAN_TILE - 1) / SCAN_TILE), nullptr, nullptr, nullptr};
+        CHK(scan_pair<T>(c, up, ScanArgs<T>{}, next));
+    }
+    KLAUNCH(c, "k_scan_tile", (k_scan_tile<T, false>), (a.nb + b.nb, BLOCK, 0), a, b);
     return UC_OK;
+}
+
+template <typename T>
+ScanArgs<T> scan_args(const T *in, T *out, uint64_t n, T *total, T *total2 = nullptr)
+{
+    return ScanArgs<T>{in, out, n, (uint32_t)((n + SCAN_TILE - 1) / SCAN_TILE), nullptr, total, total2};
 }
 
 // exclusive scan of n values; the total goes to d_total and, when given, to
@@ -3367,7 +3552,7 @@ int scan_excl(uc_ctx *c, const T *in, T *out, uint64_t n, T *d_total, DBuf &tmp,
         return UC_OK;
     }
     CHK(ensure(c, tmp, scan_scratch<T>(n) + 256));
-    return scan_level<T>(c, in, out, n, d_total, d_total2, reinterpret_cast<char *>(tmp.p));
+    return scan_pair<T>(c, scan_args(in, out, n, d_total, d_total2), ScanArgs<T>{}, reinterpret_cast<char *>(tmp.p));
 }
 
 int select_dev(uc_ctx *c)
@@ -4032,10 +4217,10 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     // totals at hist[hb] and xhist[T], and side by side in the counters for one read
     CHK(ensure(c, c->small, C_WORDS * 4));
     uint32_t *cnt = P<uint32_t>(c->small);
-    CHK(scan_excl<uint32_t>(c, P<uint32_t>(c->hist), P<uint32_t>(c->hist), hb, P<uint32_t>(c->hist) + hb, c->scan_tmp,
-                            cnt + C_TOT));
-    CHK(scan_excl<uint32_t>(c, P<uint32_t>(c->xhist), P<uint32_t>(c->xhist), T, P<uint32_t>(c->xhist) + T,
-                            c->scan_tmp, cnt + C_TOT + 1));
+    CHK(ensure(c, c->scan_tmp, scan_scratch<uint32_t>(hb) + scan_scratch<uint32_t>(T) + 256));
+    CHK(scan_pair<uint32_t>(c, scan_args<uint32_t>(P<uint32_t>(c->hist), P<uint32_t>(c->hist), hb, P<uint32_t>(c->hist) + hb, cnt + C_TOT),
+                            scan_args<uint32_t>(P<uint32_t>(c->xhist), P<uint32_t>(c->xhist), T, P<uint32_t>(c->xhist) + T, cnt + C_TOT + 1),
+                            reinterpret_cast<char *>(c->scan_tmp.p)));
     // A whole small job (lazy_sizes) does not read the totals here: the
     // buffers and grids below take the bounds x <= n and m <= 2n, the kernels
     // that need m or x read them on the device, and the host reads them with
@@ -4336,15 +4521,21 @@ int prepare_edges(uc_ctx *c)
     if (G) {
         // the oversized count is kept after the group offsets: one read for both
         uint32_t *gfd = P<uint32_t>(c->gfirst);
-        CHK(fill<uint32_t>(c, gfd + G + 1, 1, 0u));
-        KLAUNCH(c, "k_plan_count", k_plan_count, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->fboff),
-                P<uint32_t>(c->cbfirst), group_max, gfd, P<uint32_t>(c->over), gfd + G + 1);
-        CHK(scan_excl<uint32_t>(c, gfd, gfd, G, gfd + G, c->scan_tmp));
-        // (sizes the bucketing left on the device come along: placements, crossings)
         const bool pend = c->sizes_pending;
-        KLAUNCH(c, "k_plan_write", k_plan_write, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->fboff),
-                P<uint32_t>(c->cbfirst), group_max, gfd, P<EGroup>(c->egroups), pend ? cnt + C_TOT : nullptr,
-                gfd + G + 2);
+        const uint64_t S1 = c->set_sub[0];
+        if (c->n_sets == 1 && G * ((S1 + PLAN_RUN - 1) / PLAN_RUN) <= PLAN_ONE_NT) {
+            KLAUNCH(c, "k_plan_one", k_plan_one, (1, PLAN_ONE_NT, 0), P<uint32_t>(c->fboff), (uint32_t)G, (uint32_t)S1,
+                    group_max, gfd, P<EGroup>(c->egroups), P<uint32_t>(c->over), pend ? cnt + C_TOT : nullptr);
+        } else {
+            CHK(fill<uint32_t>(c, gfd + G + 1, 1, 0u));
+            KLAUNCH(c, "k_plan_count", k_plan_count, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->fboff),
+                    P<uint32_t>(c->cbfirst), group_max, gfd, P<uint32_t>(c->over), gfd + G + 1);
+            CHK(scan_excl<uint32_t>(c, gfd, gfd, G, gfd + G, c->scan_tmp));
+            // (sizes the bucketing left on the device come along: placements, crossings)
+            KLAUNCH(c, "k_plan_write", k_plan_write, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->fboff),
+                    P<uint32_t>(c->cbfirst), group_max, gfd, P<EGroup>(c->egroups), pend ? cnt + C_TOT : nullptr,
+                    gfd + G + 2);
+        }
         gf.resize(G + 4);
         CHK(d2h(c, gf.data(), gfd, (G + (pend ? 4 : 2)) * 4));
         if (pend) {
@@ -4619,16 +4810,27 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
                     P<uint64_t>(c->tsum), P<uint64_t>(c->tcnt), tile_arg(c, T));
             return UC_OK;
         }));
-        CHK(scan_excl<uint64_t>(c, P<uint64_t>(c->tcnt), P<uint64_t>(c->tcnt), T,
-                                reinterpret_cast<uint64_t *>(cnt + C_TOT), c->scan_tmp));
         return UC_OK;
+    };
+    auto splits = [&]() -> int {
+        return scan_excl<uint64_t>(c, P<uint64_t>(c->tcnt), P<uint64_t>(c->tcnt), T,
+                                   reinterpret_cast<uint64_t *>(cnt + C_TOT), c->scan_tmp);
     };
     auto totals = [&]() -> int {
         uint64_t *ttot = reinterpret_cast<uint64_t *>(cnt + C_TOT + 2);
         return scan_excl<uint64_t>(c, P<uint64_t>(c->tsum), P<uint64_t>(c->tsum), T, ttot, c->scan_tmp);
     };
+    // small jobs rank their chains in one workgroup
+    const bool one = spec && T <= CHAIN_ONE_TILES && (m >> c->shift) <= CHAIN_ONE_LIST;
     auto spec_pass = [&]() -> int {
         CHK(walks());
+        if (one) {
+            KLAUNCH(c, "k_chain_one", k_chain_one, (1, CHAIN_ONE_NT, T * 8), P<uint32_t>(c->list), cnt,
+                    P<uint32_t>(c->hasp), P<uint32_t>(c->prevseg), P<uint64_t>(c->seg), ca, cb, P<uint32_t>(c->ulen),
+                    P<uint64_t>(c->tsum), P<uint64_t>(c->tcnt), (uint32_t)T, ct);
+            return UC_OK;
+        }
+        CHK(splits());
         uint64_t *a = ca, *b = cb;
         const uint32_t g = std::max<uint32_t>(1, std::min<uint32_t>(grid_for(m), CHAIN_BLOCKS));
         KLAUNCH(c, "k_chain_init", k_chain_init, (g, BLOCK, 0), P<uint32_t>(c->list), np, P<uint32_t>(c->prevseg),
@@ -4651,7 +4853,7 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
                                             : RETRY_SLICES;
         return UC_OK;
     };
-    if (spec && pass_graph(c)) {
+    if (spec && !one && pass_graph(c)) {  // (a small job's pass is three launches)
         // no allocation or host wait may happen inside the capture
         CHK(ensure(c, c->scan_tmp, scan_scratch<uint64_t>(T) + 256));
         const std::vector<uint64_t> key = {
@@ -4684,6 +4886,7 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
         CHK(spec_pass());
     } else {
         CHK(walks());
+        CHK(splits());
         CHK(read_counts());
         const uint32_t nl = h[C_LIST];
         if (nl) {
