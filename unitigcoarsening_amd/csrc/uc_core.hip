@@ -1543,18 +1543,20 @@ __global__ __launch_bounds__(BLOCK) void k_edge_resolve(const ETile *__restrict_
 
 // LDS groups, planned on the device: one workgroup per coarse bucket; its
 // thread j packs the fine buckets 8j .. 8j+7 in order into groups of at most
-// gmax slots (a group closes when the next fine bucket would overflow it).
+// gpack slots (a group closes when the next fine bucket would overflow it; a
+// fine bucket of more than gpack and at most gmax slots is a group alone).
 // k_plan_count counts each coarse bucket's groups (and lists the fine buckets
 // above gmax); after a scan of the counts k_plan_write lays every group out
 // in one dense list, so that the edge kernel's workgroups are all busy
 // (workgroups are dealt round-robin to the XCDs: runs of empty entries
 // between the coarse buckets had left some XCDs idle).
 constexpr uint32_t PLAN_RUN = 8;  // fine buckets per planning thread
+constexpr uint32_t GROUPS_WANTED = 512, GROUP_PACK_MIN = 256;
 static_assert(MAX_SUB <= PLAN_RUN * BLOCK, "one run of fine buckets per planning thread");
 
 __device__ __forceinline__ uint32_t pack_groups(const uint32_t *__restrict__ fboff, uint32_t f0, uint32_t v0,
-                                                uint32_t v1, uint32_t gmax, EGroup *out, uint32_t *__restrict__ over,
-                                                uint32_t *__restrict__ n_over)
+                                                uint32_t v1, uint32_t gpack, uint32_t gmax, EGroup *out,
+                                                uint32_t *__restrict__ over, uint32_t *__restrict__ n_over)
 {
     uint32_t ng = 0, gb = 0, ge = 0;
     bool open = false;
@@ -1567,7 +1569,7 @@ __device__ __forceinline__ uint32_t pack_groups(const uint32_t *__restrict__ fbo
             open = false;
             continue;
         }
-        if (open && r1 - gb <= gmax) {
+        if (open && r1 - gb <= gpack) {
             ge = r1;
         } else if (r1 == r0) {
             continue;  // an empty fine bucket opens no group
@@ -1585,15 +1587,15 @@ __device__ __forceinline__ uint32_t pack_groups(const uint32_t *__restrict__ fbo
 
 // per coarse bucket: its group count (block sum of the threads' counts)
 __global__ __launch_bounds__(BLOCK) void k_plan_count(const uint32_t *__restrict__ fboff,
-                                                      const uint32_t *__restrict__ cb_first, uint32_t gmax,
-                                                      uint32_t *__restrict__ gcount, uint32_t *__restrict__ over,
+                                                      const uint32_t *__restrict__ cb_first, uint32_t gpack,
+                                                      uint32_t gmax, uint32_t *__restrict__ gcount, uint32_t *__restrict__ over,
                                                       uint32_t *__restrict__ n_over)
 {
     __shared__ uint32_t red[WAVES];
     const uint32_t g = blockIdx.x, f0 = cb_first[g], S = cb_first[g + 1] - f0;
     // S <= MAX_SUB <= PLAN_RUN * BLOCK: one run of fine buckets per thread
     const uint32_t v0 = PLAN_RUN * threadIdx.x, v1 = v0 + PLAN_RUN < S ? v0 + PLAN_RUN : S;
-    const uint32_t ng = v0 < S ? pack_groups(fboff, f0, v0, v1, gmax, nullptr, over, n_over) : 0u;
+    const uint32_t ng = v0 < S ? pack_groups(fboff, f0, v0, v1, gpack, gmax, nullptr, over, n_over) : 0u;
     const uint32_t tot = block_reduce(ng, red);
     if (threadIdx.x == 0) gcount[g] = tot;
 }
@@ -1602,8 +1604,8 @@ __global__ __launch_bounds__(BLOCK) void k_plan_count(const uint32_t *__restrict
 // (and, when given, a copy of two counters beside the offsets, for the same
 // host read)
 __global__ __launch_bounds__(BLOCK) void k_plan_write(const uint32_t *__restrict__ fboff,
-                                                      const uint32_t *__restrict__ cb_first, uint32_t gmax,
-                                                      const uint32_t *__restrict__ gfirst,
+                                                      const uint32_t *__restrict__ cb_first, uint32_t gpack,
+                                                      uint32_t gmax, const uint32_t *__restrict__ gfirst,
                                                       EGroup *__restrict__ groups, const uint32_t *__restrict__ tot,
                                                       uint32_t *__restrict__ tot_out)
 {
@@ -1611,14 +1613,14 @@ __global__ __launch_bounds__(BLOCK) void k_plan_write(const uint32_t *__restrict
     if (tot && blockIdx.x == 0 && threadIdx.x < 2) tot_out[threadIdx.x] = tot[threadIdx.x];
     const uint32_t g = blockIdx.x, f0 = cb_first[g], S = cb_first[g + 1] - f0;
     const uint32_t v0 = PLAN_RUN * threadIdx.x, v1 = v0 + PLAN_RUN < S ? v0 + PLAN_RUN : S;
-    const uint32_t ng = v0 < S ? pack_groups(fboff, f0, v0, v1, gmax, nullptr, nullptr, nullptr) : 0u;
+    const uint32_t ng = v0 < S ? pack_groups(fboff, f0, v0, v1, gpack, gmax, nullptr, nullptr, nullptr) : 0u;
     const uint32_t incl = wave_incl_scan(ng);
     const int w = threadIdx.x / 64;
     if (__lane_id() == 63) wsum[w] = incl;
     __syncthreads();
     uint32_t base = gfirst[g] + incl - ng;
     for (int q = 0; q < w; q++) base += wsum[q];
-    if (ng) pack_groups(fboff, f0, v0, v1, gmax, groups + base, nullptr, nullptr);
+    if (ng) pack_groups(fboff, f0, v0, v1, gpack, gmax, groups + base, nullptr, nullptr);
 }
 
 // The whole plan of a small job of one set in one workgroup, a thread per run
@@ -1628,7 +1630,7 @@ __global__ __launch_bounds__(BLOCK) void k_plan_write(const uint32_t *__restrict
 constexpr int PLAN_ONE_NT = 1024;
 
 __global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__restrict__ fboff, uint32_t G, uint32_t S,
-                                                          uint32_t gmax, uint32_t *__restrict__ gfirst,
+                                                          uint32_t gpack, uint32_t gmax, uint32_t *__restrict__ gfirst,
                                                           EGroup *__restrict__ groups, uint32_t *__restrict__ over,
                                                           const uint32_t *__restrict__ tot)
 {
@@ -1639,7 +1641,7 @@ __global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__rest
     const uint32_t rp = (S + PLAN_RUN - 1) / PLAN_RUN;  // runs per coarse bucket
     const uint32_t g = threadIdx.x / rp, j = threadIdx.x % rp;
     const uint32_t v0 = j * PLAN_RUN, v1 = min(S, v0 + PLAN_RUN);
-    const uint32_t ng = g < G ? pack_groups(fboff, g * S, v0, v1, gmax, nullptr, over, &n_over) : 0u;
+    const uint32_t ng = g < G ? pack_groups(fboff, g * S, v0, v1, gpack, gmax, nullptr, over, &n_over) : 0u;
     const uint32_t incl = wave_incl_scan(ng);
     const int w = threadIdx.x / 64;
     if (__lane_id() == 63) wsum[w] = incl;
@@ -1650,7 +1652,7 @@ __global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__rest
         all += wsum[q];
     }
     if (g < G && j == 0) gfirst[g] = base;
-    if (ng) pack_groups(fboff, g * S, v0, v1, gmax, groups + base, nullptr, nullptr);
+    if (ng) pack_groups(fboff, g * S, v0, v1, gpack, gmax, groups + base, nullptr, nullptr);
     if (threadIdx.x == 0) {
         gfirst[G] = all;
         gfirst[G + 1] = n_over;
@@ -4508,6 +4510,15 @@ int prepare_edges(uc_ctx *c)
     const uint32_t load = c->opts.load_pct ? c->opts.load_pct : 50;
     const bool plain = c->opts.mode == UC_MODE_PLAIN;
     const uint32_t group_max = c->opts.group_slots ? c->opts.group_slots : LDS_GROUP;
+    // Fine buckets are packed to fewer slots when a launch would otherwise have
+    // under two groups per CU: a group's phases are a serial chain of barriers
+    // and LDS round trips (24 us at 2048 slots), and small groups of it run
+    // side by side (1 M k-mers in 16 plain launches: 27 us each in groups of
+    // 2048 slots, 14 in groups of 256; 256, 512 and 1024 groups as the line
+    // measure the same).
+    uint32_t group_pack = group_max;
+    const uint64_t per_launch = plain ? c->n / ((uint64_t)c->n_sets * c->B) : c->n;
+    while (group_pack > GROUP_PACK_MIN && per_launch / group_pack < GROUPS_WANTED) group_pack /= 2;
     const uint64_t F = c->cb_first[G];
     // groups planned on the device in one dense list: coarse bucket g's
     // groups are entries [gfirst[g], gfirst[g + 1])
@@ -4525,15 +4536,15 @@ int prepare_edges(uc_ctx *c)
         const uint64_t S1 = c->set_sub[0];
         if (c->n_sets == 1 && G * ((S1 + PLAN_RUN - 1) / PLAN_RUN) <= PLAN_ONE_NT) {
             KLAUNCH(c, "k_plan_one", k_plan_one, (1, PLAN_ONE_NT, 0), P<uint32_t>(c->fboff), (uint32_t)G, (uint32_t)S1,
-                    group_max, gfd, P<EGroup>(c->egroups), P<uint32_t>(c->over), pend ? cnt + C_TOT : nullptr);
+                    group_pack, group_max, gfd, P<EGroup>(c->egroups), P<uint32_t>(c->over), pend ? cnt + C_TOT : nullptr);
         } else {
             CHK(fill<uint32_t>(c, gfd + G + 1, 1, 0u));
             KLAUNCH(c, "k_plan_count", k_plan_count, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->fboff),
-                    P<uint32_t>(c->cbfirst), group_max, gfd, P<uint32_t>(c->over), gfd + G + 1);
+                    P<uint32_t>(c->cbfirst), group_pack, group_max, gfd, P<uint32_t>(c->over), gfd + G + 1);
             CHK(scan_excl<uint32_t>(c, gfd, gfd, G, gfd + G, c->scan_tmp));
             // (sizes the bucketing left on the device come along: placements, crossings)
             KLAUNCH(c, "k_plan_write", k_plan_write, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->fboff),
-                    P<uint32_t>(c->cbfirst), group_max, gfd, P<EGroup>(c->egroups), pend ? cnt + C_TOT : nullptr,
+                    P<uint32_t>(c->cbfirst), group_pack, group_max, gfd, P<EGroup>(c->egroups), pend ? cnt + C_TOT : nullptr,
                     gfd + G + 2);
         }
         gf.resize(G + 4);
