@@ -256,6 +256,11 @@ def words_per_kmer(k: int) -> int:
     return (k + 15) // 16
 
 
+# an uninitialised bytes object of a size (PyBytes_FromStringAndSize(NULL, n)): the text is copied straight into it
+# (into an array and from there into bytes it crossed host memory twice, half of the time of a 1 M k-mer host call)
+_new_bytes = C.PYFUNCTYPE(C.py_object, C.c_void_p, C.c_ssize_t)(("PyBytes_FromStringAndSize", C.pythonapi))
+
+
 def _check(rc, ctx=None):
     if rc != UC_OK:
         L = lib()
@@ -531,9 +536,9 @@ class Compactor:
     def text(self) -> bytes:
         L = lib()
         n = L.uc_text_size(self._ctx)
-        buf = np.empty(max(n, 1), np.uint8)
-        _check(L.uc_text_copy(self._ctx, buf.ctypes.data_as(C.c_char_p), n), self._ctx)
-        return buf[:n].tobytes()
+        out = _new_bytes(None, n)  # filled before anyone else sees it
+        _check(L.uc_text_copy(self._ctx, C.cast(C.c_char_p(out), C.c_char_p), n), self._ctx)
+        return out
 
     def text_size(self):
         return lib().uc_text_size(self._ctx)
