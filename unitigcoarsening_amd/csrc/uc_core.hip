@@ -496,8 +496,31 @@ __device__ __forceinline__ uint32_t split_code(uint32_t f, uint32_t bmask, uint3
     return (f & bmask) << (split & 0xFFu) | (f >> nbits) << ((split >> 8) & 0xFFu);
 }
 
+// a job's pass-1 tiles: a planned list (several sets), or one set's, which are
+// their index (one upload and one launch fewer)
+struct Tiles1 {
+    const BTile *list;
+    uint64_t n;
+    uint32_t tile, T, fmask, split;
+};
+__device__ __forceinline__ BTile tile_at(const Tiles1 &x, uint32_t ti)
+{
+    if (x.list) return x.list[ti];
+    BTile t;
+    const uint64_t skip = (uint64_t)ti * x.tile;
+    t.kbegin = skip;
+    t.hbase = 0;
+    t.count = (uint32_t)(x.n > skip ? (x.n - skip < x.tile ? x.n - skip : x.tile) : 0);
+    t.set = 0;
+    t.ts = x.T;
+    t.tlocal = ti;
+    t.fmask = x.fmask;
+    t.split = x.split;
+    return t;
+}
+
 template <int W, int IPT, int MODE, bool C32>
-__global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict__ kin, const BTile *__restrict__ tiles,
+__global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict__ kin, Tiles1 tiles,
                                                       LminParams p, uint32_t R, uint64_t top_mask,
                                                       void *__restrict__ bkt, uint32_t *__restrict__ hist,
                                                       uint32_t *__restrict__ xhist, uint32_t n_tiles)
@@ -507,7 +530,7 @@ __global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict
     // every bucket's histogram row, which one L2 then merges into whole lines)
     const uint32_t ti = xcd_tile(n_tiles);
     if (ti == NONE) return;
-    const BTile t = tiles[ti];
+    const BTile t = tile_at(tiles, ti);
     // fine bucket = order & (B*S - 1); its low log2(B) bits are the coarse
     // bucket.  A k-mer crosses when its two fine buckets differ (both copies
     // may then share a coarse bucket).
@@ -699,7 +722,7 @@ static_assert((F_LENT | F_BORROW) < 4, "crossing flags fit two bits");
 // (flags != nullptr: no fine sort follows) or the fine index with the flag
 // bits (sub != nullptr).
 template <int W, int IPT, bool STAGE, int NT, bool C32>
-__global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict__ kin, const BTile *__restrict__ tiles,
+__global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict__ kin, Tiles1 tiles,
                                                         uint32_t B, uint32_t nbits, uint64_t top_mask,
                                                         const void *__restrict__ bkt,
                                                         const uint32_t *__restrict__ hscan,
@@ -721,7 +744,7 @@ __global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict_
     uint16_t *gcnt = reinterpret_cast<uint16_t *>(delta + B);
     const uint32_t ti = xcd_tile(n_tiles);
     if (ti == NONE) return;
-    const BTile t = tiles[ti];
+    const BTile t = tile_at(tiles, ti);
     const uint32_t s1 = t.split >> 16;
     // all of this thread's codes and k-mers in flight at once
     uint2 codes[IPT];
@@ -903,22 +926,34 @@ __global__ void k_plan1_tiles(const uint64_t *__restrict__ set_off, const uint64
     tiles[t] = bt;
 }
 
+constexpr uint32_t CNT_CLEAR = 192, CNT_SLICE = 256;  // the counters below C_TOT, and C_SLICE (see there)
+
 // row starts: rows[set * (B << J) + row] = scanned histogram at the set's
 // first tile; a coarse bucket begins at its first row (boff), and without a
 // second pass a fine bucket is its row (fboff, when given; row_first[r + 1] >
-// row_first[r] for the rows that are one).  The slot count is *mdev when
-// given (the host has not read it), else m.
+// row_first[r] for the rows that are one; without row_first every row is).
+// One set without a plan on the device: set_hbase is null and ts its tiles.
+// The slot count is *mdev when given (the host has not read it), else m.
+// A small job's later phases find their predecessor bits (n_clear words) and
+// counters cleared here (five launches in one).
 __global__ void k_gather_boff(const uint32_t *__restrict__ hscan, const uint64_t *__restrict__ set_hbase,
                               const uint32_t *__restrict__ set_ts, uint32_t n_sets, uint32_t R, uint32_t J, uint32_t m,
                               const uint32_t *__restrict__ mdev, const uint32_t *__restrict__ row_first,
-                              uint32_t *__restrict__ rows, uint32_t *__restrict__ boff, uint32_t *__restrict__ fboff)
+                              uint32_t *__restrict__ rows, uint32_t *__restrict__ boff, uint32_t *__restrict__ fboff,
+                              uint32_t ts, uint32_t *__restrict__ clear, uint64_t n_clear,
+                              uint32_t *__restrict__ counters)
 {
     const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t G = n_sets * R;
+    if (clear) {
+        for (uint64_t i = g; i < n_clear; i += (uint64_t)gridDim.x * blockDim.x) clear[i] = 0;
+        if (g < CNT_CLEAR) counters[g] = 0;
+        if (g == CNT_CLEAR) counters[CNT_SLICE] = 0;
+    }
     uint32_t v;
     if (g < G) {
         const uint32_t s = g / R, b = g % R;
-        v = hscan[set_hbase[s] + (uint64_t)b * set_ts[s]];
+        v = set_hbase ? hscan[set_hbase[s] + (uint64_t)b * set_ts[s]] : hscan[(uint64_t)b * ts];
     } else if (g == G) {
         v = mdev ? *mdev : m;
     } else {
@@ -927,8 +962,8 @@ __global__ void k_gather_boff(const uint32_t *__restrict__ hscan, const uint64_t
     rows[g] = v;
     if (boff && !(g & ((1u << J) - 1u))) boff[g >> J] = v;
     if (fboff) {
-        const uint32_t f = row_first[g];
-        if (g == G || row_first[g + 1] > f) fboff[f] = v;
+        const uint32_t f = row_first ? row_first[g] : g;
+        if (!row_first || g == G || row_first[g + 1] > f) fboff[f] = v;
     }
 }
 
@@ -2105,6 +2140,7 @@ enum {
     C_LIST = 0, C_ERR = 32, C_ACTIVE = 64, C_NONCONV = 96, C_CYC = 128, C_CUT = 160, C_TOT = 192,
     C_SLICE = 256, C_WORDS = 288
 };
+static_assert(CNT_CLEAR == C_TOT && CNT_SLICE == C_SLICE, "k_gather_boff clears the counters but the totals");
 
 // chain rounds launched before the host looks at the active counters; a
 // chain of up to 2^(SPEC_ROUNDS - 1) sampled segments converges within them
@@ -3096,6 +3132,9 @@ struct uc_ctx {
     // (lazy_sizes), and m and x hold their bounds until the edge plan's read
     // (sizes_pending)
     bool lazy_sizes = false, sizes_pending = false;
+    // the bucketing has cleared the predecessor bits / the counters already
+    bool hasp_clear = false, cnt_clear = false;
+    bool timed = false;  // emission records the job's last phase boundary
     char *pin[2] = {nullptr, nullptr};
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
     bool pin_used[2] = {false, false};
@@ -3642,7 +3681,7 @@ void reset_job(uc_ctx *c)
 {
     c->loaded = c->bucketed = c->edged = c->coarsened = c->emitted = false;
     c->edges_ready = c->no_slices = c->deferred = c->lists_spent = false;
-    c->lazy_sizes = c->sizes_pending = false;
+    c->lazy_sizes = c->sizes_pending = c->hasp_clear = c->cnt_clear = false;
     c->n_unitigs = c->n_cycles = c->text_bytes = c->n_splitters = 0;
     c->chain_rounds = 0;
     c->m = c->x = c->largest = 0;
@@ -4095,6 +4134,10 @@ int check_placements(uc_ctx *c, uint64_t n, uint64_t x)
 }
 
 constexpr uint64_t FINE_CAPPED_MAX = 1700;
+// k-mers of a job in small pass-1 tiles (bucketing of 10 k k-mers 34 -> 20 us,
+// 123 k 40 -> 27, 380 k 50 -> 41, 915 k 108 -> 99; above, the histogram has as
+// many entries as the tiles have k-mers)
+constexpr uint64_t TILE1_SMALL_MAX = 1ull << 20;
 
 // fine bits that pass 1 takes (see split_bits): all of them when the fine
 // buckets are at most MAX_BUCKETS (no second pass: seven launches fewer, 100 k
@@ -4147,9 +4190,10 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     const uint32_t R = B << J;                                    // pass-1 rows per set
     const uint32_t s1max = std::max(smax >> J, 1u);               // most fine buckets of a row
     const bool any_fine = s1max > 1;                              // a second pass follows
-    // k-mers per bucketing tile
-    constexpr int IPT1 = W == 1 ? 8 : 4;
-    const uint32_t tile1 = IPT1 * BLOCK;
+    // k-mers per bucketing tile: small jobs take small ones, so that they
+    // spread over the CUs
+    constexpr uint32_t TILE1 = (W == 1 ? 8 : 4) * BLOCK, TILE1_SMALL = 512;
+    const uint32_t tile1 = c->n <= TILE1_SMALL_MAX ? TILE1_SMALL : TILE1;
     c->tile1 = tile1;
     // tiles: every set gets at least one (possibly empty) tile so each bucket
     // row has a start in the histogram; the tiles are filled on the device
@@ -4196,15 +4240,22 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     std::memcpy(up.data() + w_cbf, set_plan.data(), w_plan * 8);
     std::memcpy(up.data() + w_cbf + w_plan, set_hbase.data(), S * 8);
     std::memcpy(up.data() + w_cbf + w_plan + w_hb, set_ts.data(), S * 4);
+    // (one set in one pass: its kernels need no plan, nor does k_plan_one)
+    const bool bare = S == 1 && !any_fine;
     CHK(ensure(c, c->cbfirst, up.size() * 8));
-    CHK(h2d(c, c->cbfirst.p, up.data(), up.size() * 8));
+    if (!bare) CHK(h2d(c, c->cbfirst.p, up.data(), up.size() * 8));
     const uint64_t *sp = P<uint64_t>(c->cbfirst) + w_cbf;
     const uint64_t *sethb = sp + w_plan;
     const uint32_t *setts = reinterpret_cast<const uint32_t *>(sethb + w_hb);
     const uint32_t *row_first = J ? reinterpret_cast<const uint32_t *>(sethb + w_hb + w_ts) : P<uint32_t>(c->cbfirst);
-    CHK(ensure(c, c->tiles, T * sizeof(BTile)));
-    KLAUNCH(c, "k_plan1_tiles", k_plan1_tiles, (grid_for(T), BLOCK, 0), sp, sp + S + 1,
-            reinterpret_cast<const uint32_t *>(sp + 2 * (uint64_t)S + 2), S, B, J, tile1, T, P<BTile>(c->tiles));
+    Tiles1 tiles{nullptr, c->n, tile1, (uint32_t)T, B * c->set_sub[0] - 1,
+                 split_bits((uint32_t)__builtin_ctz(c->set_sub[0]), J)};
+    if (S > 1) {
+        CHK(ensure(c, c->tiles, T * sizeof(BTile)));
+        KLAUNCH(c, "k_plan1_tiles", k_plan1_tiles, (grid_for(T), BLOCK, 0), sp, sp + S + 1,
+                reinterpret_cast<const uint32_t *>(sp + 2 * (uint64_t)S + 2), S, B, J, tile1, T, P<BTile>(c->tiles));
+        tiles.list = P<BTile>(c->tiles);
+    }
     CHK(ensure(c, c->hist, (hb + 1) * 4));
     CHK(ensure(c, c->xhist, (T + 1) * 4));
 
@@ -4226,9 +4277,15 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     // both fine codes of a k-mer in one word when every code fits 16 bits
     const bool c32 = (uint64_t)R * s1max <= 65536;
     CHK(ensure(c, c->bkt, std::max<uint64_t>(c->n, 1) * (c32 ? 4 : 8)));
+#define UC_CNT_(IPT, MODE, C32)                                                                                    \
+    KLAUNCH(c, "k_lmin_count", (k_lmin_count<W, IPT, MODE, C32>), (xcd_grid(T), BLOCK, (R + 1) * 4), kin, tiles, p, R, \
+            c->top_mask, c->bkt.p, P<uint32_t>(c->hist), P<uint32_t>(c->xhist), tile_arg_xcd(T))
 #define UC_CNT(MODE, C32)                                                                                          \
-    KLAUNCH(c, "k_lmin_count", (k_lmin_count<W, IPT1, MODE, C32>), (xcd_grid(T), BLOCK, (R + 1) * 4), kin,        \
-            P<BTile>(c->tiles), p, R, c->top_mask, c->bkt.p, P<uint32_t>(c->hist), P<uint32_t>(c->xhist), tile_arg_xcd(T))
+    if (tile1 == TILE1) {                                                                                          \
+        UC_CNT_(TILE1 / BLOCK, MODE, C32);                                                                         \
+    } else {                                                                                                       \
+        UC_CNT_(TILE1_SMALL / BLOCK, MODE, C32);                                                                   \
+    }
     switch (lmin_mode(l, table != nullptr)) {
     case LM_TABLE:
         if (c32) { UC_CNT(LM_TABLE, true); } else { UC_CNT(LM_TABLE, false); }
@@ -4241,6 +4298,7 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         break;
     }
 #undef UC_CNT
+#undef UC_CNT_
     // totals at hist[hb] and xhist[T], and side by side in the counters for one read
     CHK(ensure(c, c->small, C_WORDS * 4));
     uint32_t *cnt = P<uint32_t>(c->small);
@@ -4285,15 +4343,20 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     constexpr int NT1 = 512;
     const bool stage1 = !(c->opts.flags & UC_FLAG_DIRECT_SCATTER) &&
                         lmin_stage_bytes<W>(R, tile1, keep_src) <= c->lds_limit;
-#define UC_S1(ST, C32)                                                                                              \
+#define UC_S1_(IPT, ST, C32)                                                                                       \
     do {                                                                                                           \
         const size_t lds = ST ? lmin_stage_bytes<W>(R, tile1, keep_src) : lmin_lds_bytes(R, tile1 / 64);              \
-        CHK(allow_lds(c, k_lmin_scatter<W, IPT1 * BLOCK / NT1, ST, NT1, C32>, lds));                                \
-        KLAUNCH(c, "k_lmin_scatter", (k_lmin_scatter<W, IPT1 * BLOCK / NT1, ST, NT1, C32>), (xcd_grid(T), NT1, lds), \
-                kin, P<BTile>(c->tiles), R, nbits, c->top_mask, c->bkt.p, P<uint32_t>(c->hist),                     \
-                P<uint32_t>(c->xhist), P<uint64_t>(k1), any_fine ? nullptr : P<uint8_t>(c->flags),                  \
-                keep_src ? P<uint32_t>(s1) : nullptr, P<uint32_t>(c->pair_h), P<uint32_t>(c->pair_b),               \
-                any_fine ? P<uint16_t>(c->sub) : nullptr, tile_arg_xcd(T));                                         \
+        CHK(allow_lds(c, k_lmin_scatter<W, IPT, ST, NT1, C32>, lds));                                              \
+        KLAUNCH(c, "k_lmin_scatter", (k_lmin_scatter<W, IPT, ST, NT1, C32>), (xcd_grid(T), NT1, lds), kin, tiles, R,   \
+                nbits, c->top_mask, c->bkt.p, P<uint32_t>(c->hist), P<uint32_t>(c->xhist), P<uint64_t>(k1),         \
+                any_fine ? nullptr : P<uint8_t>(c->flags), keep_src ? P<uint32_t>(s1) : nullptr,                    \
+                P<uint32_t>(c->pair_h), P<uint32_t>(c->pair_b), any_fine ? P<uint16_t>(c->sub) : nullptr,           \
+                tile_arg_xcd(T));                                                                                  \
+    } while (0)
+#define UC_S1(ST, C32)                                                                                             \
+    do {                                                                                                           \
+        if (tile1 == TILE1) UC_S1_(TILE1 / NT1, ST, C32);                                                          \
+        else UC_S1_(TILE1_SMALL / NT1, ST, C32);                                                                   \
     } while (0)
     if (stage1) {
         if (c32) UC_S1(true, true);
@@ -4303,12 +4366,18 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         else UC_S1(false, false);
     }
 #undef UC_S1
+#undef UC_S1_
     // the fine rows are pass 1's rows when no second pass follows
     CHK(ensure(c, c->fboff, (F + 1) * 4));
     uint32_t *rows = J ? P<uint32_t>(c->rows) : P<uint32_t>(c->boff);
-    KLAUNCH(c, "k_gather_boff", k_gather_boff, (grid_for(GR + 1), BLOCK, 0), P<uint32_t>(c->hist), sethb, setts, S, R, J,
-            (uint32_t)c->m, mdev, row_first, rows, J ? P<uint32_t>(c->boff) : nullptr,
-            any_fine ? nullptr : P<uint32_t>(c->fboff));
+    const uint64_t hw = (c->m + 31) / 32;
+    if (lazy) CHK(ensure(c, c->hasp, hw * 4 + 8));
+    KLAUNCH(c, "k_gather_boff", k_gather_boff,
+            (grid_for(std::max<uint64_t>(std::max<uint64_t>(GR, CNT_CLEAR) + 1, lazy ? hw / 4 : 0)), BLOCK, 0),
+            P<uint32_t>(c->hist), bare ? nullptr : sethb, setts, S, R, J, (uint32_t)c->m, mdev, bare ? nullptr : row_first,
+            rows, J ? P<uint32_t>(c->boff) : nullptr, any_fine ? nullptr : P<uint32_t>(c->fboff), (uint32_t)T,
+            lazy ? P<uint32_t>(c->hasp) : nullptr, hw, cnt);
+    c->hasp_clear = c->cnt_clear = lazy;
     c->rows_valid = false;
     if (c->opts.flags & UC_FLAG_LOW_MEMORY) {
         // the codes, the input and the tile histogram are read by pass 1 and
@@ -4632,7 +4701,7 @@ int prepare_edges(uc_ctx *c)
     }
     CHK(ensure(c, c->stasks, std::max<size_t>(slices.size(), 1) * sizeof(SliceTask)));
     if (!slices.empty()) CHK(h2d(c, c->stasks.p, slices.data(), slices.size() * sizeof(SliceTask)));
-    CHK(fill<uint32_t>(c, cnt + C_SLICE, 1, 0u));
+    if (!c->cnt_clear) CHK(fill<uint32_t>(c, cnt + C_SLICE, 1, 0u));
     CHK(ensure(c, c->bgroups, std::max<size_t>(big.size(), 1) * sizeof(EGroup)));
     if (!big.empty()) CHK(h2d(c, c->bgroups.p, big.data(), big.size() * sizeof(EGroup)));
     c->n_big = big.size();
@@ -4686,7 +4755,8 @@ int prepare_edges(uc_ctx *c)
     CHK(ensure(c, c->rec, c->m * 8 + 16));
     CHK(ensure(c, c->rch, c->m + 16));
     // has-predecessor bits: every bucket sets only its own slots' bits
-    CHK(fill<uint32_t>(c, P<uint32_t>(c->hasp), (c->m + 31) / 32, 0u));
+    if (!c->hasp_clear) CHK(fill<uint32_t>(c, P<uint32_t>(c->hasp), (c->m + 31) / 32, 0u));
+    c->hasp_clear = false;
     c->n_fallback = NF;
     c->n_groups = F;
     c->bucket_done.assign(G, 0);
@@ -4835,10 +4905,15 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
     uint32_t *cnt = P<uint32_t>(c->small);
     const uint32_t *np = cnt + C_LIST;
     uint64_t *ca = P<uint64_t>(c->chainA), *cb = P<uint64_t>(c->chainB);
+    // small jobs rank their chains in one workgroup
+    const bool one = spec && T <= CHAIN_ONE_TILES && (m >> c->shift) <= CHAIN_ONE_LIST;
+    // (the bucketing cleared the counters of a small job's first pass)
+    const bool cleared = one && c->cnt_clear;
+    c->cnt_clear = false;
     // walks, the splitter/run scan, then (spec) chain ranking and the
     // unitig-length scan; everything up to the counter read
     auto walks = [&]() -> int {
-        CHK(fill<uint32_t>(c, cnt, C_SLICE, 0u));  // (the edge phase's slice flag stays)
+        if (!cleared) CHK(fill<uint32_t>(c, cnt, C_SLICE, 0u));  // (the edge phase's slice flag stays)
         CHK(with_ct(ct, [&](auto CT) -> int {
             KLAUNCH(c, "k_seg_count", k_seg_count<CT.value>, (xcd_grid(T), CT_NT, 0), P<uint64_t>(c->rec),
                     P<uint32_t>(c->hasp), P<uint8_t>(c->flags), m, c->salt, c->shift, P<uint64_t>(c->seg),
@@ -4856,8 +4931,6 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
         uint64_t *ttot = reinterpret_cast<uint64_t *>(cnt + C_TOT + 2);
         return scan_excl<uint64_t>(c, P<uint64_t>(c->tsum), P<uint64_t>(c->tsum), T, ttot, c->scan_tmp);
     };
-    // small jobs rank their chains in one workgroup
-    const bool one = spec && T <= CHAIN_ONE_TILES && (m >> c->shift) <= CHAIN_ONE_LIST;
     auto spec_pass = [&]() -> int {
         CHK(walks());
         if (one) {
@@ -5184,6 +5257,7 @@ int run_emit(uc_ctx *c)
                 P<uint32_t>(c->mcnt), P<uint32_t>(c->ulen), P<uint64_t>(c->tsum), m, ct,
                 reinterpret_cast<const uint64_t *>(cnt + C_TOT + 2), P<uint64_t>(c->setoff), gate, (uint32_t)c->n);
     }
+    if (c->timed) HIPCHK(c, hipEventRecord(c->ev[4], c->stream));
     return c->deferred ? finish_deferred(c) : set_ranges(c);
 }
 
@@ -5276,8 +5350,11 @@ bool can_defer(const uc_ctx *c)
 int timed_phases(uc_ctx *c, uint32_t l)
 {
     c->held_peak = c->held - c->pool.cap + c->pool.used;  // bytes in use, not the pool's reserve
-    for (auto &e : c->ev)
-        if (!e) HIPCHK(c, hipEventCreate(&e));
+    // (the inner boundaries only take times; the last one also publishes the
+    // results)
+    for (int i = 0; i < 5; i++)
+        if (!c->ev[i])
+            HIPCHK(c, hipEventCreateWithFlags(&c->ev[i], i < 4 ? hipEventDisableSystemFence : hipEventDefault));
     HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
     c->lazy_sizes = lazy_sizes_ok(c);
     const int rb = do_bucketize(c, l, nullptr);
@@ -5288,8 +5365,10 @@ int timed_phases(uc_ctx *c, uint32_t l)
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     CHK(do_coarsen(c, can_defer(c)));
     HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
-    CHK(do_emit(c));
-    HIPCHK(c, hipEventRecord(c->ev[4], c->stream));
+    c->timed = true;
+    const int re = do_emit(c);  // (records the last boundary after its kernels, before its reads)
+    c->timed = false;
+    CHK(re);
     HIPCHK(c, hipEventSynchronize(c->ev[4]));
     float t[4];
     for (int i = 0; i < 4; i++) HIPCHK(c, hipEventElapsedTime(&t[i], c->ev[i], c->ev[i + 1]));
