@@ -2615,22 +2615,54 @@ __device__ __forceinline__ void put_kmer(char *o, uint64_t at, const Kmer<W> &x,
     for (; i < k; i++) o[i] = base_char(char_at<W>(x, i));
 }
 
-// the same at any LDS address: whole words (LDS takes them unaligned), the last
-// one over the end of the one before, so that every lane does the same k / 4
-// stores
+// the same into LDS: up to three bytes to the first 4-byte boundary, aligned
+// words, up to three bytes after them, every lane in the same steps (the word
+// count differs by one between lanes).  Unaligned LDS words need no steps at
+// the ends, but LDS takes them one lane a cycle: 300 us of LDS time on the 50
+// Mbp job.
 template <int W>
-__device__ __forceinline__ void put_kmer_lds(char *o, const Kmer<W> &x, uint32_t k)
+__device__ __forceinline__ void put_kmer_lds(char *o, uint64_t at, const Kmer<W> &x, uint32_t k)
 {
-    auto word = [&](uint32_t i) {
-        const uint32_t v = kmer_chars4<W>(x, i);
-        __builtin_memcpy(o + i, &v, 4);
-    };
-    uint32_t i = 0;
-    for (; i + 4 <= k; i += 4) word(i);
-    if (i < k && k >= 4)
-        word(k - 4);
-    else
-        for (; i < k; i++) o[i] = base_char(char_at<W>(x, i));
+    if (k < 8) {  // (uniform)
+        put_kmer<W>(o, at, x, k);
+        return;
+    }
+    const uint32_t lead = (0u - (uint32_t)at) & 3u, sh = 2 * lead;
+    uint32_t d[2 * W + 1];
+#pragma unroll
+    for (int j = 0; j < 2 * W; j++) d[j] = (uint32_t)(x.w[j / 2] >> (32 * (j % 2)));
+    d[2 * W] = 0;
+    const uint32_t first = chars4(d[0]);
+    if (lead > 0) o[0] = (char)first;
+    if (lead > 1) o[1] = (char)(first >> 8);
+    if (lead > 2) o[2] = (char)(first >> 16);
+    // the rest from the boundary on
+#pragma unroll
+    for (int j = 0; j < 2 * W; j++) d[j] = __builtin_amdgcn_alignbit(d[j + 1], d[j], sh);
+    o += lead;
+    const uint32_t whole = (k - 3) / 4;  // words that every lane has
+    uint32_t tail = 0;                   // the byte of codes after them
+#pragma unroll
+    for (int q = 0; q < 8 * W; q++) {
+        const uint32_t b = d[q / 4] >> (8 * (q % 4));
+        if ((uint32_t)q < whole)  // (uniform)
+            *reinterpret_cast<uint32_t *>(o + 4 * q) = chars4(b);
+        else if ((uint32_t)q == whole)
+            tail = (q % 4 == 3 ? b & 0xFFu : b) | (q % 4 == 3 && q / 4 + 1 < 2 * W ? d[q / 4 + 1] << 8 : 0u);
+    }
+    // up to six characters are left
+    o += 4 * whole;
+    uint32_t left = k - lead - 4 * whole;
+    uint32_t c = chars4(tail);
+    if (left >= 4) {
+        *reinterpret_cast<uint32_t *>(o) = c;
+        c = chars4(tail >> 8);
+        o += 4;
+        left -= 4;
+    }
+    if (left > 0) o[0] = (char)c;
+    if (left > 1) o[1] = (char)(c >> 8);
+    if (left > 2) o[2] = (char)(c >> 16);
 }
 
 // byte i (0..15) of a 16-byte line
@@ -2795,7 +2827,7 @@ __global__ __launch_bounds__(CT_NT) void k_head_emit(const uint64_t *__restrict_
             // (the bytes of runs after a head's first run are written later
             // over what the stage holds there)
             if (h) {
-                put_kmer_lds<W>(stg + (off - a), x, k);
+                put_kmer_lds<W>(stg + (off - a), off, x, k);
                 put_rest(stg + (off - a) + k, r, rch, s);
             }
             wave_sync();
