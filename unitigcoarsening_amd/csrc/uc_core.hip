@@ -215,34 +215,59 @@ __device__ __forceinline__ uint32_t lmer_order(uint32_t code, const LminParams &
 // lmin_buckets.h:67-94: minimum order over the l-mers of the (k-1)-prefix
 // (o1) and of the (k-1)-suffix (o2); the l-mer code keeps its first
 // character most significant.  Both share the middle l-mers: o1 = min(first,
-// middle), o2 = min(middle, last).  Characters are read 16 to a 32-bit word;
-// the loop over a word's characters keeps a run-time (uniform) trip count, so
-// the code stays small whatever k is.
+// middle), o2 = min(middle, last).  With the k-mer's characters in reverse
+// order (character i at bits 64 W - 2 - 2 i), the l-mer at character i is the
+// word's bits from 64 W - 2 (i + l) on, under the characters before it: one
+// funnel shift of two 32-bit words, where a rolling code takes an extract and
+// a shift-or (and l steps to fill it).  Two l-mers at a time share one
+// three-input minimum.  The loops' trip counts are uniform, so the code stays
+// small whatever k is.
 template <int W, int MODE>
 __device__ __forceinline__ void double_lmin(const Kmer<W> &x, const LminParams &p, uint32_t &o1, uint32_t &o2)
 {
     const uint32_t k = p.k, l = p.l;
-    uint32_t lmer = 0, mid = NONE;
-    // characters [i0, i1) into the rolling code; hash (into mid) when HASH
-    auto scan = [&](uint32_t i0, uint32_t i1, auto hash) {
+    uint32_t r[2 * W + 1];  // reversed characters, lowest word first
 #pragma unroll
-        for (int q = 0; q < 2 * W; q++) {
-            const uint32_t b = 16u * q;
-            const uint32_t lo = i0 > b ? i0 : b, hi = i1 < b + 16u ? i1 : b + 16u;
-            const uint32_t w = (uint32_t)(x.w[q / 2] >> (32 * (q % 2)));
-#pragma unroll 1
-            for (uint32_t i = lo; i < hi; i++) {  // uniform trip count
-                // characters older than the l-mer stay above its 2l bits
-                lmer = (lmer << 2) | __builtin_amdgcn_ubfe(w, 2 * (i - b), 2);
-                if constexpr (decltype(hash)::value) mid = min(mid, lmer_order_m<MODE>(lmer, p));
+    for (int j = 0; j < W; j++) {
+        const uint64_t y = rev_chars64(x.w[W - 1 - j]);
+        r[2 * j] = (uint32_t)y;
+        r[2 * j + 1] = (uint32_t)(y >> 32);
+    }
+    r[2 * W] = 0;
+    // bit positions: the first l-mer's, and the last one's below it
+    const uint32_t top = 64 * W - 2 * l, bot = 64 * W - 2 * k;
+    uint32_t mid = NONE, first = 0, last = 0;
+#pragma unroll
+    for (int q = 2 * W - 1; q >= 0; q--) {
+        // l-mers whose position lies in word q: bits [lo, hi) of it, from the top
+        const uint32_t b = 32u * q;
+        if (bot >= b + 32u || top < b) continue;
+        auto code = [&](uint32_t at) { return __builtin_amdgcn_alignbit(r[q + 1], r[q], at); };
+        uint32_t at = (top < b + 30u ? top : b + 30u) - b;  // positions are even
+        const uint32_t end = (bot > b ? bot : b) - b;        // the lowest one here
+        if (top - b == at) {
+            first = lmer_order_m<MODE>(code(at), p);
+            if (at == end) {  // (k - 1 >= l: the last l-mer is another one, in the next word)
+                continue;
             }
+            at -= 2;
         }
-    };
-    scan(0, l, std::false_type{});
-    const uint32_t first = lmer_order_m<MODE>(lmer, p);
-    scan(l, k - 1, std::true_type{});
-    scan(k - 1, k, std::false_type{});
-    const uint32_t last = lmer_order_m<MODE>(lmer, p);
+        uint32_t stop = end;  // the lowest middle one: the last l-mer is not in the middle
+        if (bot >= b) {
+            last = lmer_order_m<MODE>(code(bot - b), p);
+            stop = bot - b + 2;
+        }
+        // middle l-mers at at, at - 2, ..., stop
+        int32_t n = ((int32_t)at - (int32_t)stop) / 2 + 1;
+        if ((int32_t)at < (int32_t)stop) n = 0;
+#pragma unroll 1
+        for (; n >= 2; n -= 2) {
+            const uint32_t u = lmer_order_m<MODE>(code(at), p), v = lmer_order_m<MODE>(code(at - 2), p);
+            mid = min(mid, min(u, v));
+            at -= 4;
+        }
+        if (n) mid = min(mid, lmer_order_m<MODE>(code(at), p));
+    }
     o1 = min(first, mid);
     o2 = min(mid, last);
 }
