@@ -589,25 +589,35 @@ __global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict
     if (threadIdx.x == 0) xhist[ti] = cnt[R];
 }
 
-// lanes whose home (mp) or borrow (ms) placement goes to bucket v
-__device__ __forceinline__ void match_bucket(uint32_t v, uint32_t nbits, uint64_t V, uint64_t C,
-                                             const uint64_t *BP, const uint64_t *BS, uint64_t &mp, uint64_t &ms)
+// LDS writes of one wave visible to the whole wave (no block barrier)
+__device__ __forceinline__ void wave_sync()
 {
-    mp = V;
-    ms = C;
-#pragma unroll
-    for (int j = 0; j < 10; j++) {
-        if ((uint32_t)j < nbits) {
-            if ((v >> j) & 1u) {
-                mp &= BP[j];
-                ms &= BS[j];
-            } else {
-                mp &= ~BP[j];
-                ms &= ~BS[j];
-            }
-        }
-    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+
+// the lanes where p holds (the builtin compares straight into a scalar pair;
+// __ballot goes through an int and back)
+__device__ __forceinline__ uint64_t lanes_of(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+// bits of a mask below this lane, added to n
+__device__ __forceinline__ uint32_t below(uint64_t mask, uint32_t n)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, n));
+}
+
+// One bit of the lanes' bucket numbers: the lanes with it (B) keep or leave a
+// lane's matching set by its own bit (m: all ones or zero), a three-input op
+// per half.  Every match below runs bit by bit with all its sets in registers:
+// a loop over a uniform bit count, no arrays of lane masks (which spilled) and
+// no branch per bit.
+__device__ __forceinline__ uint64_t match_bit(uint64_t set, uint64_t B, uint32_t m)
+{
+    const uint32_t lo = (uint32_t)set & ~((uint32_t)B ^ m), hi = (uint32_t)(set >> 32) & ~((uint32_t)(B >> 32) ^ m);
+    return (uint64_t)lo | ((uint64_t)hi << 32);
+}
+__device__ __forceinline__ uint32_t bit_mask(uint32_t v, uint32_t q) { return (uint32_t)__builtin_amdgcn_sbfe((int)v, q, 1); }
 
 // block_excl_scan_n for PER = 2 or 4 values per thread at an aligned array:
 // each thread's values move as one 8- or 16-byte word and stay in registers
@@ -797,49 +807,46 @@ __global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict_
     __syncthreads();
     block_excl_scan_n<NT>(tstart, B, wsum);
     for (uint32_t v = threadIdx.x; v < B; v += NT) delta[v] -= tstart[v];
-    const int lane = __lane_id(), w = threadIdx.x / 64;
-    const uint64_t lt = (1ull << lane) - 1ull, me = 1ull << lane;
+    const int w = threadIdx.x / 64;
     // 1. every item's rank among its wave's placements of the same bucket
     // (homes before borrows within a lane), and each wave's count per bucket
+    // (the placement that none comes before writes it)
     uint32_t rh[IPT], rb[IPT], rc[IPT];
 #pragma unroll
     for (int j = 0; j < IPT; j++) {
         rh[j] = rb[j] = rc[j] = 0;
         if ((uint32_t)j * NT >= t.count) break;  // uniform over the block
         const uint32_t idx = (uint32_t)j * NT + threadIdx.x;
-        const bool valid = idx < t.count;
-        uint32_t bp = 0, bs = 0;
-        bool cross = false;
-        if (valid) {
-            bp = codes[j].x >> s1;
-            bs = codes[j].y >> s1;
-            cross = codes[j].x != codes[j].y;
-        }
-        const uint64_t V = __ballot(valid), C = __ballot(cross);
-        uint64_t BP[10], BS[10];
-#pragma unroll
-        for (int q = 0; q < 10; q++) {
-            BP[q] = (uint32_t)q < nbits ? (uint64_t)__ballot(valid && ((bp >> q) & 1u)) : 0ull;
-            BS[q] = (uint32_t)q < nbits ? (uint64_t)__ballot(cross && ((bs >> q) & 1u)) : 0ull;
-        }
-        // placements of lower lanes in the same bucket: homes (hp*) and borrows (hs*)
+        const bool valid = idx < t.count, cross = valid && codes[j].x != codes[j].y;
+        const uint32_t bp = codes[j].x >> s1, bs = codes[j].y >> s1;
+        // homes (hp) and borrows (hs) in this lane's home bucket, and in its borrow's
+        const uint64_t V = lanes_of(valid), C = lanes_of(cross);
+        uint64_t hp = V, hs = C, gp = V, gs = C;
         uint16_t *gc = gcnt + (size_t)(j * NW + w) * (B + 1);
-        if (valid) {
-            uint64_t hp = 0, hs = 0;
-            match_bucket(bp, nbits, V, C, BP, BS, hp, hs);
-            const uint64_t M = hp | hs;
-            if ((M & (0ull - M)) == me) gc[bp] = (uint16_t)(__popcll(hp) + __popcll(hs));
-            rh[j] = (uint32_t)(__popcll(hp & lt) + __popcll(hs & lt));
+        if (C) {  // uniform over the wave
+            for (uint32_t q = 0; q < nbits; q++) {
+                const uint32_t mp = bit_mask(bp, q), ms = bit_mask(bs, q);
+                const uint64_t BP = lanes_of(mp != 0), BS = lanes_of(ms != 0);
+                hp = match_bit(hp, BP, mp);
+                hs = match_bit(hs, BS, mp);
+                gp = match_bit(gp, BP, ms);
+                gs = match_bit(gs, BS, ms);
+            }
+            if (cross) {
+                const uint32_t r = below(gs, below(gp, 0));
+                if (r == 0) gc[bs] = (uint16_t)(__popcll(gp) + __popcll(gs));
+                rb[j] = r + (bp == bs ? 1u : 0u);
+                rc[j] = below(C, 0);
+                if (rc[j] == 0) gc[B] = (uint16_t)__popcll(C);
+            }
+        } else {
+            for (uint32_t q = 0; q < nbits; q++) {
+                const uint32_t mp = bit_mask(bp, q);
+                hp = match_bit(hp, lanes_of(mp != 0), mp);
+            }
         }
-        if (cross) {
-            uint64_t hp = 0, hs = 0;
-            match_bucket(bs, nbits, V, C, BP, BS, hp, hs);
-            const uint64_t M = hp | hs;
-            if ((M & (0ull - M)) == me) gc[bs] = (uint16_t)(__popcll(hp) + __popcll(hs));
-            rb[j] = (uint32_t)(__popcll(hp & lt) + __popcll(hs & lt)) + (bp == bs ? 1u : 0u);
-            rc[j] = (uint32_t)__popcll(C & lt);
-        }
-        if (C && (C & (0ull - C)) == me) gc[B] = (uint16_t)__popcll(C);
+        rh[j] = below(hs, below(hp, 0));
+        if (valid && rh[j] == 0) gc[bp] = (uint16_t)(__popcll(hp) + __popcll(hs));
     }
     __syncthreads();
     // 2. each column's exclusive prefix over the groups in tile order
@@ -1230,8 +1237,6 @@ __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ ti
     uint32_t *ssrc = reinterpret_cast<uint32_t *>(st + (size_t)TILE * 8 * W);
     uint16_t *ssub = reinterpret_cast<uint16_t *>(st + (size_t)TILE * 8 * W + (src ? (size_t)TILE * 4 : 0));
     const int lane = __lane_id(), w = threadIdx.x / 64;
-    const uint64_t lt = (1ull << lane) - 1ull, me = 1ull << lane;
-    const uint64_t zero[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const uint32_t c0 = (uint32_t)w * CHUNK;
     uint32_t *mywc = wc + (uint32_t)w * S;
     // the tile's base in every fine bucket
@@ -1292,21 +1297,25 @@ __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ ti
 #pragma unroll
         for (int j = 0; j < IPT; j++) {
             const bool valid = vf[j] != NONE;
-            const uint64_t V = __ballot(valid);
-            if (!V) break;  // uniform over the wave
+            uint64_t M = lanes_of(valid);
+            if (!M) break;  // uniform over the wave
             const uint32_t v = vf[j] & SUB_MASK;
-            uint64_t BP[10];
-#pragma unroll
-            for (int q = 0; q < 10; q++) BP[q] = (uint32_t)q < nbits ? (uint64_t)__ballot(valid && ((v >> q) & 1u)) : 0ull;
-            uint64_t M = 0, none;
-            match_bucket(v, nbits, V, 0ull, BP, zero, M, none);
-            uint32_t old = 0;
-            if (valid && (M & (0ull - M)) == me) old = atomicAdd(&mywc[v], (uint32_t)__popcll(M));
-            const int leader = valid ? __builtin_ctzll(M) : lane;
-            const uint32_t base = __shfl(old, leader, 64);
+            for (uint32_t q = 0; q < nbits; q++) {
+                const uint32_t m = bit_mask(v, q);
+                M = match_bit(M, lanes_of(m != 0), m);
+            }
+            // the wave's base in the bucket moves past the group (its last lane
+            // writes it; a wave's LDS accesses keep their order)
+            const uint32_t rank = below(M, 0), size = (uint32_t)__popcll(M);
+            uint32_t base = 0;
+            if (valid) {
+                base = mywc[v];
+                if (rank + 1 == size) mywc[v] = base + size;
+            }
+            wave_sync();
             if (valid) {
                 const uint64_t s = t.kbegin + r0 + c0 + 64u * j + (uint32_t)lane;
-                const uint32_t li = base + (uint32_t)__popcll(M & lt);
+                const uint32_t li = base + rank;
                 const uint32_t ns = delta[v] + li;
                 if constexpr (STAGE) {
                     skm[li] = xs[j];
@@ -2104,14 +2113,6 @@ __global__ __launch_bounds__(1024) void k_edge_slice(const uint64_t *__restrict_
 // splitter (one step per run: its length and the next run), and chains of
 // segments are ranked by pointer jumping over the sampled splitters only.
 // Emission then walks each segment again, copying its runs' characters.
-
-// LDS writes of one wave visible to the whole wave (no block barrier)
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Slots per contraction (and emission) tile: the fewest, from CT_MIN to
 // CT_MAX, whose tiles one scan workgroup takes, so that small jobs spread over
