@@ -144,6 +144,23 @@ __device__ __forceinline__ void key_hash(const Kmer<W> &x, uint32_t &h, uint32_t
     }
 }
 
+// position of a key in an LDS table of 2^(32 - shift) entries: the high bits
+// of a multiplicative hash, a multiply per word and one more (32-bit multiplies
+// run at a quarter of the rate; key_hash takes one more per word)
+template <int W>
+__device__ __forceinline__ uint32_t lds_hash(const Kmer<W> &x, uint32_t shift)
+{
+    uint32_t t = (uint32_t)x.w[0] + (uint32_t)(x.w[0] >> 32) * 0x9E3779B1u;
+    t ^= t >> 16;
+    if constexpr (W == 2) {
+        t = t * 0x85EBCA6Bu + (uint32_t)x.w[1];
+        t ^= t >> 15;
+        t = t * 0xC2B2AE35u + (uint32_t)(x.w[1] >> 32);
+        t ^= t >> 16;
+    }
+    return (t * 0x85EBCA77u) >> shift;
+}
+
 // lexicographic key: reverse the order of the 2-bit characters
 __device__ __forceinline__ uint64_t rev_chars64(uint64_t x)
 {
@@ -1774,9 +1791,12 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
     const EGroup gr = groups[blockIdx.x];
     const uint32_t n = gr.end - gr.begin;
     if (n == 0) return;  // an unused group entry
-    uint32_t tcap = 64;
-    while (tcap < 2 * n) tcap <<= 1;
-    const uint32_t tmask = tcap - 1;
+    uint32_t tcap = 64, tshift = 26;
+    while (tcap < 2 * n) {
+        tcap <<= 1;
+        tshift--;
+    }
+    const uint32_t tmask = tcap - 1, last = n - 1;
     const uint32_t off0 = gr.begin & 31;
     const uint32_t nw = (off0 + n + 31) / 32;
     // the thread's k-mers stay in registers through insert and lookup; every
@@ -1810,29 +1830,33 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
         hpos[e] = NONE;
         if (i < n && !((fs >> (8 * e)) & F_BORROW)) {
-            uint32_t h, tag;
-            key_hash<W>(prefix_key<W>(xs[e], pm0, pm1), h, tag);
-            hpos[e] = h & tmask;
+            hpos[e] = lds_hash<W>(prefix_key<W>(xs[e], pm0, pm1), tshift);
         }
     }
     __syncthreads();
-    // prefixes of home copies
+    // Prefixes of home copies.  The probe loops have one exit and no branch
+    // inside: the occupant's k-mer is read whether or not there is one (any
+    // staged slot does for an empty entry).  A CU has one scalar unit, and the
+    // masks of nested branches kept it busier than the vector units (323 M
+    // scalar against 268 M vector instructions on the 50 Mbp job).  A table
+    // holds at most half as many keys as entries, so every probe ends.
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
         if (hpos[e] == NONE) continue;
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
         const Kmer<W> key = prefix_key<W>(xs[e], pm0, pm1);
-        uint32_t pos = hpos[e];
-        for (uint32_t probe = 0; probe < tcap; probe++) {
+        uint32_t pos = hpos[e], at;
+        bool same;
+        uint32_t cur;
+        do {
             if (CNT) np++;
-            const uint32_t cur = atomicCAS(&tab[pos], LDS_EMPTY, i);
-            if (cur == LDS_EMPTY) break;
-            if (key_eq<W>(prefix_key<W>(km[cur & 0xFFFFu], pm0, pm1), key)) {
-                atomicOr(&tab[pos], LDS_SHARED);
-                break;
-            }
+            at = pos;
+            cur = atomicCAS(&tab[at], LDS_EMPTY, i);
+            const Kmer<W> other = km[min(cur & 0xFFFFu, last)];
+            same = key_eq<W>(prefix_key<W>(other, pm0, pm1), key);
             pos = (pos + 1) & tmask;
-        }
+        } while ((cur != LDS_EMPTY) & !same);
+        if (cur != LDS_EMPTY) atomicOr(&tab[at], LDS_SHARED);
     }
     // lookup positions (suffixes of every copy that carries its out-edge here)
 #pragma unroll
@@ -1840,9 +1864,7 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
         hpos[e] = NONE;
         if (i < n && !((fs >> (8 * e)) & F_LENT)) {
-            uint32_t h, tag;
-            key_hash<W>(suffix_key<W>(xs[e]), h, tag);
-            hpos[e] = h & tmask;
+            hpos[e] = lds_hash<W>(suffix_key<W>(xs[e]), tshift);
         }
     }
     __syncthreads();
@@ -1853,17 +1875,19 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
         uint16_t hp = LDS_NOHIT;
         if (hpos[e] != NONE) {
             const Kmer<W> key = suffix_key<W>(xs[e]);
-            uint32_t pos = hpos[e];
-            for (uint32_t probe = 0; probe < tcap; probe++) {
+            uint32_t pos = hpos[e], at, en;
+            bool same;
+            do {
                 if (CNT) np++;
-                const uint32_t en = tab[pos];
-                if (en == LDS_EMPTY) break;
-                if (key_eq<W>(prefix_key<W>(km[en & 0xFFFFu], pm0, pm1), key)) {
-                    atomicAdd(&tab[pos], 1u << 24);
-                    hp = (uint16_t)pos;
-                    break;
-                }
+                at = pos;
+                en = tab[at];
+                const Kmer<W> other = km[min(en & 0xFFFFu, last)];
+                same = key_eq<W>(prefix_key<W>(other, pm0, pm1), key);
                 pos = (pos + 1) & tmask;
+            } while ((en != LDS_EMPTY) & !same);
+            if (en != LDS_EMPTY) {
+                atomicAdd(&tab[at], 1u << 24);
+                hp = (uint16_t)at;
             }
         }
         hitp[i] = hp;
@@ -1935,7 +1959,7 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
         for (;;) {
             pd[v] = i | (d << 16);
             const uint16_t nx = succ[v];
-            if (nx == LDS_NOHIT || d + 1 >= n) break;
+            if ((nx == LDS_NOHIT) | (d + 1 >= n)) break;
             v = nx;
             d++;
         }
