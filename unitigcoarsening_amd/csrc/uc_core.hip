@@ -126,6 +126,20 @@ __device__ __forceinline__ bool key_eq(const Kmer<W> &a, const Kmer<W> &b)
         return a.w[0] == b.w[0] && a.w[1] == b.w[1];
 }
 
+// zero when the (k-1)-prefix of x is key (one three-input op per 32 bits)
+template <int W>
+__device__ __forceinline__ uint32_t prefix_diff(const Kmer<W> &x, const Kmer<W> &key, uint64_t pm0, uint64_t pm1)
+{
+    uint32_t d = 0;
+#pragma unroll
+    for (int j = 0; j < 2 * W; j++) {
+        const uint64_t pm = j < 2 ? pm0 : pm1;
+        const uint32_t a = (uint32_t)(x.w[j / 2] >> (32 * (j % 2))), b = (uint32_t)(key.w[j / 2] >> (32 * (j % 2)));
+        d |= __builtin_amdgcn_bitop3_b32(a, b, (uint32_t)(pm >> (32 * (j % 2))), 0x28);  // (a ^ b) & mask
+    }
+    return d;
+}
+
 // table position hash and an independent 28-bit tag
 template <int W>
 __device__ __forceinline__ void key_hash(const Kmer<W> &x, uint32_t &h, uint32_t &tag)
@@ -1759,7 +1773,7 @@ __global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__rest
 //   LDS layout (nb = launch capacity, a power of two):
 //     km   Kmer<W>[nb]   staged k-mers
 //     tab  uint32[2nb]   owner (16 bits) | LDS_SHARED | hits << 24, or LDS_EMPTY
-//     hitp uint16[nb]    table position of each slot's suffix hit
+//     predl uint16[nb]   run predecessor of each slot
 //     hb   uint32[nb/32 + 2]  has-predecessor bits, aligned to global words
 
 constexpr uint32_t LDS_EMPTY = 0xFFFFFFFFu;
@@ -1771,6 +1785,11 @@ __host__ __device__ constexpr size_t edge_lds_bytes(uint32_t nb)
 {
     return (size_t)nb * (8 * W + 8 + 2) + ((size_t)nb / 32 + 2) * 4;
 }
+
+// keeps a value that a loop leaves behind in its vector register: a condition
+// on it after the loop would otherwise be carried through every round as a lane
+// mask (three scalar instructions)
+__device__ __forceinline__ void opaque(uint32_t &v) { asm volatile("" : "+v"(v)); }
 
 template <int W, int EB, int GMAX, bool CNT>
 __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ kmer, const EGroup *__restrict__ groups,
@@ -1786,7 +1805,7 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
     extern __shared__ __align__(16) unsigned char lds[];
     Kmer<W> *km = reinterpret_cast<Kmer<W> *>(lds);
     uint32_t *tab = reinterpret_cast<uint32_t *>(lds + (size_t)nb * 8 * W);
-    uint16_t *hitp = reinterpret_cast<uint16_t *>(lds + (size_t)nb * (8 * W + 8));
+    uint16_t *predl = reinterpret_cast<uint16_t *>(lds + (size_t)nb * (8 * W + 8));
     uint32_t *hb = reinterpret_cast<uint32_t *>(lds + (size_t)nb * (8 * W + 10));  // nb is a multiple of 64
     const EGroup gr = groups[blockIdx.x];
     const uint32_t n = gr.end - gr.begin;
@@ -1800,25 +1819,28 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
     const uint32_t off0 = gr.begin & 31;
     const uint32_t nw = (off0 + n + 31) / 32;
     // the thread's k-mers stay in registers through insert and lookup; every
-    // load is in flight before the first LDS store
+    // load is in flight before the first LDS store (items past the end load
+    // the last slot: no branch, and no wait for one item's flags before the
+    // next one's loads)
     static_assert(EPT <= 8, "one flag byte per item in a 64-bit word");
     Kmer<W> xs[EPT];
-    uint64_t fs = 0;  // flag byte of item e at bits 8e
+    uint32_t fl[EPT];
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
-        const uint32_t i = threadIdx.x + (uint32_t)e * EB;
-        if (i < n) {
-            xs[e] = load_kmer<W>(kmer, gr.begin + i, ~0ull);
-            fs |= (uint64_t)flags[gr.begin + i] << (8 * e);
-        }
+        const uint32_t g = gr.begin + min(threadIdx.x + (uint32_t)e * EB, last);
+        xs[e] = load_kmer<W>(kmer, g, ~0ull);
+        fl[e] = flags[g];
     }
+    uint64_t fs = 0;  // flag byte of item e at bits 8e (past the end: neither inserted, looked up nor walked)
     uint32_t lc = 0;  // last character of item e at bits 2e
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
+        fs |= (uint64_t)(i < n ? fl[e] : (uint32_t)(F_BORROW | F_LENT)) << (8 * e);
+        lc |= char_at<W>(xs[e], k - 1) << (2 * e);
         if (i < n) {
             km[i] = xs[e];
-            lc |= char_at<W>(xs[e], k - 1) << (2 * e);
+            predl[i] = LDS_NOHIT;
         }
     }
     for (uint32_t i = threadIdx.x; i < tcap; i += EB) tab[i] = LDS_EMPTY;
@@ -1827,11 +1849,8 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
     uint32_t hpos[EPT];
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
-        const uint32_t i = threadIdx.x + (uint32_t)e * EB;
-        hpos[e] = NONE;
-        if (i < n && !((fs >> (8 * e)) & F_BORROW)) {
-            hpos[e] = lds_hash<W>(prefix_key<W>(xs[e], pm0, pm1), tshift);
-        }
+        const uint32_t h = lds_hash<W>(prefix_key<W>(xs[e], pm0, pm1), tshift);
+        hpos[e] = (fs >> (8 * e)) & F_BORROW ? NONE : h;
     }
     __syncthreads();
     // Prefixes of home copies.  The probe loops have one exit and no branch
@@ -1845,52 +1864,45 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
         if (hpos[e] == NONE) continue;
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
         const Kmer<W> key = prefix_key<W>(xs[e], pm0, pm1);
-        uint32_t pos = hpos[e], at;
-        bool same;
-        uint32_t cur;
+        uint32_t pos = hpos[e], at, cur, more;
         do {
             if (CNT) np++;
             at = pos;
             cur = atomicCAS(&tab[at], LDS_EMPTY, i);
-            const Kmer<W> other = km[min(cur & 0xFFFFu, last)];
-            same = key_eq<W>(prefix_key<W>(other, pm0, pm1), key);
+            more = min(cur + 1u, prefix_diff<W>(km[min(cur & 0xFFFFu, last)], key, pm0, pm1));
             pos = (pos + 1) & tmask;
-        } while ((cur != LDS_EMPTY) & !same);
+        } while (more);  // neither empty (cur + 1 = 0) nor the same key
+        opaque(cur);
         if (cur != LDS_EMPTY) atomicOr(&tab[at], LDS_SHARED);
     }
     // lookup positions (suffixes of every copy that carries its out-edge here)
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
-        const uint32_t i = threadIdx.x + (uint32_t)e * EB;
-        hpos[e] = NONE;
-        if (i < n && !((fs >> (8 * e)) & F_LENT)) {
-            hpos[e] = lds_hash<W>(suffix_key<W>(xs[e]), tshift);
-        }
+        const uint32_t h = lds_hash<W>(suffix_key<W>(xs[e]), tshift);
+        hpos[e] = (fs >> (8 * e)) & F_LENT ? NONE : h;
     }
     __syncthreads();
+    uint16_t hit[EPT];  // table position of the item's suffix hit
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
-        const uint32_t i = threadIdx.x + (uint32_t)e * EB;
-        if (i >= n) continue;
         uint16_t hp = LDS_NOHIT;
         if (hpos[e] != NONE) {
             const Kmer<W> key = suffix_key<W>(xs[e]);
-            uint32_t pos = hpos[e], at, en;
-            bool same;
+            uint32_t pos = hpos[e], at, en, more;
             do {
                 if (CNT) np++;
                 at = pos;
                 en = tab[at];
-                const Kmer<W> other = km[min(en & 0xFFFFu, last)];
-                same = key_eq<W>(prefix_key<W>(other, pm0, pm1), key);
+                more = min(en + 1u, prefix_diff<W>(km[min(en & 0xFFFFu, last)], key, pm0, pm1));
                 pos = (pos + 1) & tmask;
-            } while ((en != LDS_EMPTY) & !same);
+            } while (more);
+            opaque(en);
             if (en != LDS_EMPTY) {
                 atomicAdd(&tab[at], 1u << 24);
                 hp = (uint16_t)at;
             }
         }
-        hitp[i] = hp;
+        hit[e] = hp;
     }
     __syncthreads();
     // keep u -> v when v's prefix is unshared and was hit exactly once; the
@@ -1901,7 +1913,7 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
         tgt[e] = LDS_NOHIT;
         if (i >= n) continue;
-        const uint16_t hp = hitp[i];
+        const uint16_t hp = hit[e];
         uint32_t l = NO_LINK;
         if (hp != LDS_NOHIT) {
             const uint32_t en = tab[hp];
@@ -1920,11 +1932,8 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
         const uint32_t bits = hb[j];
         if (bits) atomicOr(&hasp[(gr.begin >> 5) + j], bits);
     }
-    // runs: run predecessor of every slot (hitp is free now; the flags and
-    // last characters stay in registers, so the k-mer staging area is free)
-    uint16_t *predl = hitp;
-    for (uint32_t i = threadIdx.x; i < n; i += EB) predl[i] = LDS_NOHIT;
-    __syncthreads();
+    // runs: run predecessor of every slot (the flags and last characters stay
+    // in registers, so the k-mer staging area is free)
 #pragma unroll
     for (int e = 0; e < EPT; e++)
         if (tgt[e] != LDS_NOHIT) predl[tgt[e]] = (uint16_t)(threadIdx.x + (uint32_t)e * EB);
@@ -1954,15 +1963,17 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
     for (int e = 0; e < EPT; e++) {
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
         rl[e] = 0;
-        if (i >= n || ((fs >> (8 * e)) & F_BORROW) || predl[i] != LDS_NOHIT) continue;
+        if ((fs >> (8 * e)) & F_BORROW) continue;
+        if (predl[i] != LDS_NOHIT) continue;
         uint32_t v = i, d = 0;
-        for (;;) {
+        uint32_t more;
+        do {
             pd[v] = i | (d << 16);
-            const uint16_t nx = succ[v];
-            if ((nx == LDS_NOHIT) | (d + 1 >= n)) break;
-            v = nx;
+            v = succ[v];
+            more = min(v ^ (uint32_t)LDS_NOHIT, n - 1 - d);  // (d < n: n slots bound the walk)
             d++;
-        }
+        } while (more);
+        d--;
         rl[e] = (uint16_t)(d + 1);
         sc[i] = d + 1;
     }
@@ -1972,7 +1983,7 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
-        if (i < n && !((fs >> (8 * e)) & F_BORROW) && pd[i] == LDS_EMPTY) sc[i] = 1;
+        if (!((fs >> (8 * e)) & F_BORROW) && pd[i] == LDS_EMPTY) sc[i] = 1;
     }
     __syncthreads();
     block_excl_scan_n<EB>(sc, n, wsum);
