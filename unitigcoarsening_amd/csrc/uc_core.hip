@@ -593,12 +593,15 @@ __global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict
     for (uint32_t i = threadIdx.x; i <= R; i += BLOCK) cnt[i] = 0;
     __syncthreads();
     const uint32_t bmask = p.B - 1, nbits = (uint32_t)__builtin_ctz(p.B), s1 = t.split >> 16;
-    // all of this thread's k-mers in flight at once
+    // all of this thread's k-mers in flight at once (threads past the end load
+    // the last one: a branch per item would wait for each load in turn)
     Kmer<W> xs[IPT];
+    if (t.count) {
 #pragma unroll
-    for (int j = 0; j < IPT; j++) {
-        const uint32_t idx = (uint32_t)j * BLOCK + threadIdx.x;
-        if (idx < t.count) xs[j] = load_kmer<W>(kin, t.kbegin + idx, top_mask);
+        for (int j = 0; j < IPT; j++) {
+            const uint32_t idx = min((uint32_t)j * BLOCK + threadIdx.x, t.count - 1);
+            xs[j] = load_kmer<W>(kin, t.kbegin + idx, top_mask);
+        }
     }
 #pragma unroll
     for (int j = 0; j < IPT; j++) {
@@ -815,14 +818,14 @@ __global__ __launch_bounds__(NT) void k_lmin_scatter(const uint64_t *__restrict_
     // all of this thread's codes and k-mers in flight at once
     uint2 codes[IPT];
     Kmer<W> xs[IPT];
+    // (threads past the end load the last one: a branch per item would wait
+    // for each load in turn)
+    if (t.count == 0) return;  // an empty set's tile
 #pragma unroll
     for (int j = 0; j < IPT; j++) {
-        const uint32_t idx = (uint32_t)j * NT + threadIdx.x;
-        codes[j] = make_uint2(0u, 0u);
-        if (idx < t.count) {
-            codes[j] = get_codes<C32>(bkt, t.kbegin + idx);
-            xs[j] = load_kmer<W>(kin, t.kbegin + idx, top_mask);
-        }
+        const uint64_t at = t.kbegin + min((uint32_t)j * NT + threadIdx.x, t.count - 1);
+        codes[j] = get_codes<C32>(bkt, at);
+        xs[j] = load_kmer<W>(kin, at, top_mask);
     }
     {
         uint32_t *g32 = reinterpret_cast<uint32_t *>(gcnt);
@@ -1147,11 +1150,11 @@ __global__ __launch_bounds__(SUB_COUNT_NT) void k_sub_count(const uint16_t *__re
 #pragma unroll
         for (int j = 0; j < PER; j++) {
             const uint32_t i = i0 + (uint32_t)j * SUB_COUNT_NT + threadIdx.x;
-            v[j] = i < t.count ? (uint32_t)sub[t.kbegin + i] & SUB_MASK : NONE;
+            v[j] = sub[t.kbegin + min(i, t.count - 1)];
         }
 #pragma unroll
         for (int j = 0; j < PER; j++)
-            if (v[j] != NONE) atomicAdd(&cnt[v[j]], 1u);
+            if (i0 + (uint32_t)j * SUB_COUNT_NT + threadIdx.x < t.count) atomicAdd(&cnt[v[j] & SUB_MASK], 1u);
     }
     __syncthreads();
     for (uint32_t v = threadIdx.x; v < S; v += SUB_COUNT_NT) hist[t.hbase + (uint64_t)t.tlocal * S + v] = cnt[v];
@@ -1255,7 +1258,7 @@ __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ ti
     if (ti == NONE) return;
     const BTile t = tiles[ti];
     const uint32_t S = t.fmask;
-    if (S == 0) return;  // past the last tile
+    if (S == 0 || t.count == 0) return;  // past the last tile, or a row without slots
     const uint32_t nbits = (uint32_t)__builtin_ctz(S);
     const bool src = sin != nullptr;
     uint32_t *wc = reinterpret_cast<uint32_t *>(lds);  // NW x S
@@ -1280,20 +1283,23 @@ __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ ti
     auto load_round = [&](uint32_t r0, uint32_t *V, Kmer<W> *X, uint32_t *R) {
 #pragma unroll
         for (int j = 0; j < IPT; j++) {
-            const uint32_t idx = r0 + c0 + 64u * j + (uint32_t)lane;
-            V[j] = NONE;
+            // (past the end: the last slot, without a branch)
+            const uint64_t s = t.kbegin + min(r0 + c0 + 64u * j + (uint32_t)lane, t.count - 1);
+            V[j] = (uint32_t)sub[s];
+            X[j] = load_kmer<W>(kin, s, ~0ull);
+        }
+#pragma unroll
+        for (int j = 0; j < IPT; j++) {
             R[j] = 0;
-            if (idx < t.count) {
-                const uint64_t s = t.kbegin + idx;
-                V[j] = (uint32_t)sub[s];
-                X[j] = load_kmer<W>(kin, s, ~0ull);
-                if (src) R[j] = sin[s];
-            }
+            if (src) R[j] = sin[t.kbegin + min(r0 + c0 + 64u * j + (uint32_t)lane, t.count - 1)];
         }
     };
     load_round(0, vf, xs, sr);
     for (uint32_t r0 = 0; r0 < t.count; r0 += TILE) {  // uniform over the block
         if (r0 + TILE < t.count) load_round(r0 + TILE, nvf, nxs, nsr);
+#pragma unroll
+        for (int j = 0; j < IPT; j++)
+            if (r0 + c0 + 64u * j + (uint32_t)lane >= t.count) vf[j] = NONE;
         for (uint32_t i = threadIdx.x; i < NW * S; i += NT) wc[i] = 0;
         __syncthreads();
         // 1. per-wave counts
@@ -2259,15 +2265,17 @@ __global__ __launch_bounds__(CT_NT) void k_seg_count(const uint64_t *__restrict_
     const uint32_t ti = xcd_tile(n_tiles);
     if (ti == NONE) return;
     const uint64_t base = (uint64_t)ti * CT;
-    // flags and has-predecessor words of this thread's slots, all in flight
-    // at once (the flag array has slack past its end, so no load is guarded)
-    uint8_t f[ITEMS];
-    uint32_t hw[ITEMS];
+    // flags, has-predecessor words and run records of this thread's slots, all
+    // in flight at once (past the end: the last slot, without a branch; a slot
+    // that starts no run has no record, and its word is not used)
+    uint32_t f[ITEMS], hw[ITEMS];
+    uint64_t first[ITEMS];
 #pragma unroll
     for (int j = 0; j < ITEMS; j++) {
-        const uint64_t s = base + (uint64_t)j * NT + threadIdx.x;
-        f[j] = s < m ? flags[s] : (uint8_t)F_BORROW;
-        hw[j] = hasp[(s < m ? s : 0) >> 5];
+        const uint32_t s = (uint32_t)min(base + (uint64_t)j * NT + threadIdx.x, (uint64_t)m - 1);
+        f[j] = flags[s];
+        hw[j] = hasp[s >> 5];
+        first[j] = rec[s];
     }
     // splitters; sampled ones get list slots with one atomic per tile
     bool hd[ITEMS], rd[ITEMS];
@@ -2275,17 +2283,13 @@ __global__ __launch_bounds__(CT_NT) void k_seg_count(const uint64_t *__restrict_
 #pragma unroll
     for (int j = 0; j < ITEMS; j++) {
         const uint32_t s = (uint32_t)(base + (uint64_t)j * NT + threadIdx.x);
-        const bool cand = (f[j] & (F_BORROW | F_RUNHEAD)) == F_RUNHEAD;
+        const bool cand = s < m && (f[j] & (F_BORROW | F_RUNHEAD)) == F_RUNHEAD;
         hd[j] = cand && !((hw[j] >> (s & 31)) & 1u);
         rd[j] = cand && !hd[j] && sampled(s, salt, shift);
         nruns += cand;
         nr += rd[j];
         nh += hd[j];
     }
-    // every head's first run record in flight at once
-    uint64_t first[ITEMS];
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) first[j] = hd[j] ? rec[base + (uint64_t)j * NT + threadIdx.x] : 0ull;
     uint64_t acc = (uint64_t)nh << 32;
     uint32_t nm = 0;
 #pragma unroll
@@ -2813,13 +2817,15 @@ __global__ __launch_bounds__(CT_NT) void k_head_emit(const uint64_t *__restrict_
     // slot's flags, predecessor bit and run record, all in flight at once
     const uint32_t nml = mcnt[ti];
     const uint64_t tb = tile_off[ti];
-    uint32_t fh[CTI];
+    // (past the end: the last slot, without a branch)
+    uint32_t fh[CTI], hw[CTI];
     uint64_t hr[CTI];
 #pragma unroll
     for (int j = 0; j < CTI; j++) {
-        const uint64_t s = t0 + (uint64_t)j * NT + threadIdx.x;
-        fh[j] = s < m ? (uint32_t)flags[s] | (((hasp[s >> 5] >> (s & 31)) & 1u) << 8) : (uint32_t)F_BORROW;
-        hr[j] = s < m ? rec[s] : 0ull;
+        const uint32_t s = (uint32_t)min(t0 + (uint64_t)j * NT + threadIdx.x, (uint64_t)m - 1);
+        fh[j] = flags[s];
+        hw[j] = hasp[s >> 5];
+        hr[j] = rec[s];
     }
     uint64_t ml[CTI];
 #pragma unroll
@@ -2833,8 +2839,9 @@ __global__ __launch_bounds__(CT_NT) void k_head_emit(const uint64_t *__restrict_
     uint32_t nh = 0;
 #pragma unroll
     for (int j = 0; j < CTI; j++) {
-        const bool h = !(fh[j] & (F_BORROW | 0x100u));
-        const uint64_t mask = __ballot(h);
+        const uint32_t s = (uint32_t)t0 + j * NT + lane;
+        const bool h = s < m && !(fh[j] & F_BORROW) && !((hw[j] >> (s & 31)) & 1u);
+        const uint64_t mask = lanes_of(h);
         if (lane == 0) {
             hmask[j] = mask;
             gbase[j] = nh;
