@@ -1390,13 +1390,37 @@ __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ ti
 
 // (the pair count is *xdev when given: the host has not read it, and x is
 // then its bound)
-__global__ void k_pair_remap(uint32_t *__restrict__ pair_home, uint32_t *__restrict__ pair_borrow, uint32_t x,
-                             const uint32_t *__restrict__ xdev, const uint32_t *__restrict__ perm)
+constexpr int PAIR_ITEMS = 4;  // pairs per thread: their random reads are in flight together
+
+__global__ __launch_bounds__(BLOCK) void k_pair_remap(uint32_t *__restrict__ pair_home, uint32_t *__restrict__ pair_borrow,
+                                                      uint32_t x, const uint32_t *__restrict__ xdev,
+                                                      const uint32_t *__restrict__ perm)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= x || (xdev && i >= *xdev)) return;
-    pair_home[i] = perm[pair_home[i]];
-    pair_borrow[i] = perm[pair_borrow[i]];
+    const uint32_t n = xdev ? min(x, *xdev) : x, i0 = blockIdx.x * (PAIR_ITEMS * BLOCK) + threadIdx.x;
+    if (i0 >= n) return;
+    uint32_t h[PAIR_ITEMS], b[PAIR_ITEMS];
+#pragma unroll
+    for (int j = 0; j < PAIR_ITEMS; j++) {
+        const uint32_t i = min(i0 + (uint32_t)j * BLOCK, n - 1);
+        h[j] = pair_home[i];
+        b[j] = pair_borrow[i];
+    }
+#pragma unroll
+    for (int j = 0; j < PAIR_ITEMS; j++) {
+        const uint32_t i = i0 + (uint32_t)j * BLOCK;
+        const bool on = i < n;
+        const uint32_t v = perm[on ? h[j] : h[0]], u = perm[on ? b[j] : b[0]];
+        h[j] = v;
+        b[j] = u;
+    }
+#pragma unroll
+    for (int j = 0; j < PAIR_ITEMS; j++) {
+        const uint32_t i = i0 + (uint32_t)j * BLOCK;
+        if (i < n) {
+            pair_home[i] = h[j];
+            pair_borrow[i] = b[j];
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2066,78 +2090,92 @@ __global__ __launch_bounds__(1024) void k_edge_slice(const uint64_t *__restrict_
     const uint32_t n = t.end - t.begin;
     for (uint32_t i = threadIdx.x; i < SLICE_TAB; i += NT) tab[i] = LDS_EMPTY;
     __syncthreads();
-    // 1. prefixes of home copies in this slice
-    for (uint32_t i = threadIdx.x; i < n; i += NT) {
-        const uint32_t s = t.begin + i;
-        if (ro.flags[s] & F_BORROW) continue;
-        const Kmer<W> key = prefix_key<W>(load_kmer<W>(kmer, s, ~0ull), pm0, pm1);
-        uint32_t h, tag;
-        key_hash<W>(key, h, tag);
-        if (fastrange(h, t.P) != t.p) continue;
-        const uint32_t tg = (tag & 0x7Fu) << 17;
-        uint32_t pos = h & (SLICE_TAB - 1), probe = 0;
-        for (; probe < plimit; probe++) {
-            if (CNT) np++;
-            const uint32_t cur = atomicCAS(&tab[pos], LDS_EMPTY, i | tg);
-            if (cur == LDS_EMPTY) break;
-            if ((cur & SLICE_TAGS) == tg &&
-                key_eq<W>(prefix_key<W>(load_kmer<W>(kmer, t.begin + (cur & 0xFFFFu), ~0ull), pm0, pm1), key)) {
-                atomicOr(&tab[pos], LDS_SHARED);
-                break;
-            }
-            pos = (pos + 1) & (SLICE_TAB - 1);
+    // each sweep loads U slots per thread before it looks at one
+    constexpr int U = 4;
+    Kmer<W> xs[U];
+    uint8_t fl[U];
+    auto load = [&](uint32_t i0) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t s = t.begin + min(i0 + (uint32_t)u * NT + threadIdx.x, n - 1);
+            xs[u] = load_kmer<W>(kmer, s, ~0ull);
+            fl[u] = ro.flags[s];
         }
-        // table full (not expected at SLICE_KEYS per slice): the host runs
-        // the edge phase again with these fine buckets on HBM tables
-        if (probe == plimit) atomicOr(err, 1u);
+    };
+    // 1. prefixes of home copies in this slice
+    for (uint32_t i0 = 0; i0 < n; i0 += U * NT) {
+        load(i0);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t i = i0 + (uint32_t)u * NT + threadIdx.x;
+            const Kmer<W> key = prefix_key<W>(xs[u], pm0, pm1);
+            uint32_t h, tag;
+            key_hash<W>(key, h, tag);
+            if (i >= n || (fl[u] & F_BORROW) || fastrange(h, t.P) != t.p) continue;
+            const uint32_t tg = (tag & 0x7Fu) << 17;
+            uint32_t pos = h & (SLICE_TAB - 1), probe = 0;
+            for (; probe < plimit; probe++) {
+                if (CNT) np++;
+                const uint32_t cur = atomicCAS(&tab[pos], LDS_EMPTY, i | tg);
+                if (cur == LDS_EMPTY) break;
+                if ((cur & SLICE_TAGS) == tg &&
+                    key_eq<W>(prefix_key<W>(load_kmer<W>(kmer, t.begin + (cur & 0xFFFFu), ~0ull), pm0, pm1), key)) {
+                    atomicOr(&tab[pos], LDS_SHARED);
+                    break;
+                }
+                pos = (pos + 1) & (SLICE_TAB - 1);
+            }
+            // table full (not expected at SLICE_KEYS per slice): the host runs
+            // the edge phase again with these fine buckets on HBM tables
+            if (probe == plimit) atomicOr(err, 1u);
+        }
     }
     __syncthreads();
     // 2. suffix hits of the copies that carry their out-edge here, this slice
-    for (uint32_t i = threadIdx.x; i < n; i += NT) {
-        const uint32_t s = t.begin + i;
-        if (ro.flags[s] & F_LENT) continue;
-        const Kmer<W> key = suffix_key<W>(load_kmer<W>(kmer, s, ~0ull));
-        uint32_t h, tag, pos;
-        key_hash<W>(key, h, tag);
-        if (fastrange(h, t.P) != t.p) continue;
-        if (slice_probe<W, CNT>(tab, kmer, t.begin, key, h, (tag & 0x7Fu) << 17, pm0, pm1, pos, np))
-            atomicAdd(&tab[pos], 1u << 24);
+    for (uint32_t i0 = 0; i0 < n; i0 += U * NT) {
+        load(i0);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t i = i0 + (uint32_t)u * NT + threadIdx.x;
+            const Kmer<W> key = suffix_key<W>(xs[u]);
+            uint32_t h, tag, pos;
+            key_hash<W>(key, h, tag);
+            if (i >= n || (fl[u] & F_LENT) || fastrange(h, t.P) != t.p) continue;
+            if (slice_probe<W, CNT>(tab, kmer, t.begin, key, h, (tag & 0x7Fu) << 17, pm0, pm1, pos, np))
+                atomicAdd(&tab[pos], 1u << 24);
+        }
     }
     __syncthreads();
     // 3. links and singleton runs: a lent k-mer belongs to its prefix's
-    // slice, every other k-mer to its suffix's
-    for (uint32_t i = threadIdx.x; i < n; i += NT) {
-        const uint32_t s = t.begin + i;
-        const uint8_t f = ro.flags[s];
-        const Kmer<W> x = load_kmer<W>(kmer, s, ~0ull);
-        uint32_t h, tag;
-        if (f & F_LENT) {
-            key_hash<W>(prefix_key<W>(x, pm0, pm1), h, tag);
-            if (fastrange(h, t.P) != t.p) continue;
-            link[s] = s;  // its own run head, until the splice
-            ro.flags[s] = (uint8_t)(f | F_RUNHEAD);
-            ro.rec[s] = make_rec(NONE, 1u, s, s, char_at<W>(x, k - 1));
-            ro.rch[s] = base_char(char_at<W>(x, k - 1));
-            continue;
-        }
-        const Kmer<W> key = suffix_key<W>(x);
-        key_hash<W>(key, h, tag);
-        if (fastrange(h, t.P) != t.p) continue;
-        uint32_t l = NO_LINK;
-        uint32_t pos;
-        if (slice_probe<W, CNT>(tab, kmer, t.begin, key, h, (tag & 0x7Fu) << 17, pm0, pm1, pos, np)) {
-            const uint32_t e = tab[pos];
-            if (!(e & LDS_SHARED) && (e >> 24) == 1u) {  // unshared prefix, exactly one suffix hit
-                const uint32_t v = t.begin + (e & 0xFFFFu);
-                l = v;
-                atomicOr(&hasp[v >> 5], 1u << (v & 31));
+    // slice, every other k-mer to its suffix's (only that slice writes the
+    // slot's flags, and only bits that no slice reads)
+    for (uint32_t i0 = 0; i0 < n; i0 += U * NT) {
+        load(i0);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t i = i0 + (uint32_t)u * NT + threadIdx.x, s = t.begin + i;
+            const uint8_t f = fl[u];
+            const bool lent = f & F_LENT;
+            const Kmer<W> x = xs[u], key = lent ? prefix_key<W>(x, pm0, pm1) : suffix_key<W>(x);
+            uint32_t h, tag;
+            key_hash<W>(key, h, tag);
+            if (i >= n || fastrange(h, t.P) != t.p) continue;
+            uint32_t l = lent ? s : NO_LINK, next = NONE;  // (a lent k-mer's link: its own run head, until the splice)
+            uint32_t pos;
+            if (!lent && slice_probe<W, CNT>(tab, kmer, t.begin, key, h, (tag & 0x7Fu) << 17, pm0, pm1, pos, np)) {
+                const uint32_t e = tab[pos];
+                if (!(e & LDS_SHARED) && (e >> 24) == 1u) {  // unshared prefix, exactly one suffix hit
+                    const uint32_t v = t.begin + (e & 0xFFFFu);
+                    l = next = v;
+                    atomicOr(&hasp[v >> 5], 1u << (v & 31));
+                }
             }
-        }
-        link[s] = l;
-        if (!(f & F_BORROW)) {
-            ro.flags[s] = (uint8_t)(f | F_RUNHEAD);
-            ro.rec[s] = make_rec((uint32_t)l, 1u, s, s, char_at<W>(x, k - 1));
-            ro.rch[s] = base_char(char_at<W>(x, k - 1));
+            link[s] = l;
+            if (!(f & F_BORROW)) {
+                ro.flags[s] = (uint8_t)(f | F_RUNHEAD);
+                ro.rec[s] = make_rec(next, 1u, s, s, char_at<W>(x, k - 1));
+                ro.rch[s] = base_char(char_at<W>(x, k - 1));
+            }
         }
     }
     if (CNT) add_probes<NT>(probes, np, pred_);
@@ -2175,17 +2213,31 @@ __host__ __device__ constexpr uint32_t ct_tile(uint64_t m)
 
 // the borrowed duplicate's out-edge moves to the home copy; the target keeps
 // its has-predecessor bit
-__global__ void k_splice(const uint32_t *__restrict__ pair_home, const uint32_t *__restrict__ pair_borrow, uint32_t x,
-                         uint32_t *__restrict__ link, uint64_t *__restrict__ rec)
+__global__ __launch_bounds__(BLOCK) void k_splice(const uint32_t *__restrict__ pair_home,
+                                                  const uint32_t *__restrict__ pair_borrow, uint32_t x,
+                                                  uint32_t *__restrict__ link, uint64_t *__restrict__ rec)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= x) return;
-    const uint32_t h = pair_home[i];
-    const uint32_t l = link[pair_borrow[i]];
-    const uint32_t head = link[h];  // the lent k-mer's run head
-    link[h] = l;
-    // a lent k-mer ends its run: the run continues through the duplicate's edge
-    reinterpret_cast<uint32_t *>(rec)[2ull * head] = l;  // the record's next-run field
+    const uint32_t i0 = blockIdx.x * (PAIR_ITEMS * BLOCK) + threadIdx.x;
+    if (i0 >= x) return;
+    uint32_t h[PAIR_ITEMS], l[PAIR_ITEMS], head[PAIR_ITEMS];
+#pragma unroll
+    for (int j = 0; j < PAIR_ITEMS; j++) {  // (past the end: the first pair again)
+        const uint32_t i = i0 + (uint32_t)j * BLOCK, c = i < x ? i : i0;
+        h[j] = pair_home[c];
+        l[j] = pair_borrow[c];
+    }
+#pragma unroll
+    for (int j = 0; j < PAIR_ITEMS; j++) {
+        l[j] = link[l[j]];
+        head[j] = link[h[j]];  // the lent k-mer's run head
+    }
+#pragma unroll
+    for (int j = 0; j < PAIR_ITEMS; j++) {
+        if (i0 + (uint32_t)j * BLOCK >= x) continue;
+        link[h[j]] = l[j];
+        // a lent k-mer ends its run: the run continues through the duplicate's edge
+        reinterpret_cast<uint32_t *>(rec)[2ull * head[j]] = l[j];  // the record's next-run field
+    }
 }
 
 // list index for every flagged lane: one atomic per wave
@@ -4551,7 +4603,7 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         else UC_S2(false);
 #undef UC_S2
         if (c->x)
-            KLAUNCH(c, "k_pair_remap", k_pair_remap, (grid_for(c->x), BLOCK, 0), P<uint32_t>(c->pair_h),
+            KLAUNCH(c, "k_pair_remap", k_pair_remap, (grid_for(c->x, PAIR_ITEMS * BLOCK), BLOCK, 0), P<uint32_t>(c->pair_h),
                     P<uint32_t>(c->pair_b), (uint32_t)c->x, lazy ? cnt + C_TOT + 1 : nullptr, P<uint32_t>(c->perm));
         // pass 2's input and the permutation are dead now
         CHK(drop(c, c->kmer2));
@@ -5237,7 +5289,7 @@ int do_coarsen(uc_ctx *c, bool defer)
     c->salt = (uint32_t)(c->opts.seed * 0x9E3779B97F4A7C15ull >> 32);
     c->shift = c->opts.sample_log2 ? c->opts.sample_log2 : DEFAULT_SAMPLE_LOG2;
     if (c->x && !c->spliced) {  // (once per edge result: it consumes the lent k-mers' run heads)
-        KLAUNCH(c, "k_splice", k_splice, (grid_for(c->x), BLOCK, 0), P<uint32_t>(c->pair_h), P<uint32_t>(c->pair_b),
+        KLAUNCH(c, "k_splice", k_splice, (grid_for(c->x, PAIR_ITEMS * BLOCK), BLOCK, 0), P<uint32_t>(c->pair_h), P<uint32_t>(c->pair_b),
                 (uint32_t)c->x, P<uint32_t>(c->link), P<uint64_t>(c->rec));
     }
     c->spliced = true;
