@@ -18,15 +18,31 @@ def fine_count(n, B, fine_slots):
     return s
 
 
-# (buckets, fine_slots, set sizes): one pass with all fine bits (up to 1024 rows), two passes with the fine bits
-# split or not, sets with fewer fine bits than pass 1 takes (none, some), one set, an empty set, 1 and 1024 buckets
-@pytest.mark.parametrize("B,fine_slots,sizes", [
-    (1, 64, [12_000]), (1, 64, [90_000]), (64, 64, [5_000]), (64, 64, [60_000]), (128, 64, [9_000]),
-    (1024, 64, [3_000]), (1024, 64, [140_000]), (16, 64, [200, 9_000, 0, 2_100]), (4, 64, [40, 70_000, 300, 2_500]),
+def minima(x, k, l, order):
+    """Minimum order over the l-mers of every k-mer's (k-1)-prefix and (k-1)-suffix."""
+    code, low, ends = np.zeros(x.shape[0], np.int64), None, []
+    for i in range(k):  # (first character most significant)
+        code = (code << 2 | (x[:, i // 16].astype(np.int64) >> (2 * (i % 16))) & 3) & (4 ** l - 1)
+        if l <= i + 1 < k:
+            o = order[code]
+            ends = ends or [o]
+            low = o if i + 1 == l + 1 else low if low is None else np.minimum(low, o)
+    last = order[code]
+    return np.minimum(ends[0], low), np.minimum(low, last)
+
+
+# (k, buckets, fine_slots, set sizes): one pass with all fine bits (up to 1024 rows), two passes with the fine bits
+# split or not, sets with fewer fine bits than pass 1 takes (none, some), one set, an empty set, 1 and 1024 buckets,
+# rows long enough for the fine sort's long rounds (32 768 slots on average)
+@pytest.mark.parametrize("k,B,fine_slots,sizes", [
+    (31, 1, 64, [12_000]), (31, 1, 64, [90_000]), (31, 64, 64, [5_000]), (31, 64, 64, [60_000]), (31, 128, 64, [9_000]),
+    (31, 1024, 64, [3_000]), (31, 1024, 64, [140_000]), (63, 1024, 64, [140_000]), (63, 64, 64, [60_000]),
+    (31, 16, 64, [200, 9_000, 0, 2_100]), (31, 4, 64, [40, 70_000, 300, 2_500]),
+    (31, 2, 64, [1_150_000]), (47, 2, 64, [1_150_000]),
 ])
-def test_slots_are_the_stable_sort_by_fine_bucket(B, fine_slots, sizes):
-    k, l, seed = 31, 8, 77
-    kmers = [uc.medium_model(3 + i, max(n, 100), k)[:n] for i, n in enumerate(sizes)]
+def test_slots_are_the_stable_sort_by_fine_bucket(k, B, fine_slots, sizes):
+    l, seed = 8, 77
+    kmers = [uc.medium_model(3 + i, max(n + n // 16, 100), k)[:n] for i, n in enumerate(sizes)]
     sizes = [x.shape[0] for x in kmers]
     with uc.Compactor(n_buckets=B, seed=seed, keep_src=True, fine_slots=fine_slots) as c:
         c.load(np.concatenate(kmers), k, set_sizes=sizes)
@@ -38,11 +54,7 @@ def test_slots_are_the_stable_sort_by_fine_bucket(B, fine_slots, sizes):
     assert n_fine == B * sum(subs)
     keys, ids, want_flags, n0 = [], [], [], 0
     for s, (x, sub) in enumerate(zip(kmers, subs)):
-        # l-mer codes with the first character most significant, from the packed words
-        chars = [(x[:, i // 16].astype(np.int64) >> (2 * (i % 16))) & 3 for i in range(k)]
-        codes = [sum(chars[i + j] << (2 * (l - 1 - j)) for j in range(l)) for i in range(k - l + 1)]
-        o = [order[code] for code in codes]
-        fine = [np.minimum.reduce(o[a:b]) & (B * sub - 1) for a, b in ((0, k - l), (1, k - l + 1))]
+        fine = [o & (B * sub - 1) for o in minima(x, k, l, order)]
         slot_key = [((s * B + (f & (B - 1))) << 32) | f // B for f in fine]
         n = x.shape[0]
         cross = fine[0] != fine[1]

@@ -1217,8 +1217,8 @@ __global__ __launch_bounds__(BLOCK) void k_sub_rows(const uint32_t *__restrict__
     if (g == G - 1 && threadIdx.x == 0) fboff[cb_first[G]] = mdev ? *mdev : m;
 }
 
-// Pass-2 scatter with LDS staging.  A planned tile (up to ROUNDS rounds of
-// IPT * NT slots of one coarse bucket) is sorted round by round; each round is
+// Pass-2 scatter with LDS staging.  A planned tile (up to SUB_TILE slots of one
+// coarse bucket, in rounds of IPT * NT) is sorted round by round; each round is
 // ranked per wave: each wave owns a chunk of consecutive slots, counts its
 // slots per fine bucket (ballot groups, one LDS add per group), the counts are
 // scanned once per round, and a second sweep gives every slot its stable
@@ -1226,7 +1226,7 @@ __global__ __launch_bounds__(BLOCK) void k_sub_rows(const uint32_t *__restrict__
 // there in LDS and written out in that order, so consecutive lanes store
 // consecutive addresses of one fine bucket's run.  The running base of every
 // fine bucket carries from round to round, so the histogram holds one row per
-// planned tile (ROUNDS times fewer than one per round), and the next round's
+// planned tile (not one per round), and the next round's
 // slots are loaded while the current one is ranked.
 __host__ __device__ constexpr size_t sub_book_bytes(uint32_t S, uint32_t nw = WAVES)
 {
@@ -1239,7 +1239,8 @@ __host__ __device__ constexpr size_t sub_lds_bytes(uint32_t tile, uint32_t S, bo
     return sub_book_bytes(S, nw) + (stage ? (size_t)tile * 8 * W + (src ? (size_t)tile * 4 : 0) + (size_t)tile * 2 : 0);
 }
 
-constexpr uint32_t SUB_ROUNDS = 4;
+constexpr uint32_t SUB_TILE = 8192;   // slots of a planned fine-sort tile
+constexpr uint64_t LONG_ROW = 32768;  // average slots of a row from which rounds are long
 
 template <int W, bool STAGE, int IPT, int NT>
 __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ tiles, const uint16_t *__restrict__ sub,
@@ -4547,22 +4548,22 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     // fine buckets: stable sort of each coarse bucket's slots by fine index,
     // planned and run on the device (no host round trip)
     if (any_fine) {
-        // slots per fine-sort round; LDS staging when the device has the room
-        // (2048-slot rounds: half the LDS of 4096, so more tiles in flight per
-        // CU; measured 0.82 -> 0.71 ms for the staged one-word scatter).  A
-        // planned tile is SUB_ROUNDS rounds.
-        constexpr int IPT2 = 8;
-        // (1, 2 and 4 rounds measured 0.73, 0.71 and 0.68 ms for the count,
-        // column scan and scatter together on the 50 Mbp job: the scatter takes
-        // the same time whatever the rounds, the histogram work shrinks)
-        const uint32_t round2 = IPT2 * BLOCK, tile2 = SUB_ROUNDS * round2;
-        // (two-word k-mers measured faster unstaged here: 4.9 vs 5.5 ms on
-        // 303 M slots; one-word ones staged: 0.82 vs 0.85 ms on 53 M)
-        // threads per 2048-slot tile: 512 for the staged one-word form, 1024
-        // for the direct two-word form (each measured best of 256/512/1024)
+        // A planned tile is SUB_TILE slots, in rounds of 4096 when the rows are
+        // long (longer pieces of each fine bucket per round, fewer half-written
+        // lines) and fit LDS, else of 2048 (more workgroups per CU, which short
+        // rows need): 50 Mbp job 2805 -> 2729 us, 45 M 63-mers 3378 -> 3290, 12 M
+        // 47-mers 1089 -> 1045, but 256 sets of 5 000-slot rows 4643 -> 4706.
+        // 512 threads for one-word k-mers, 1024 for two-word ones (each best of
+        // 256, 512 and 1024); both staged in LDS.
+        constexpr uint32_t R_SHORT = 2048, R_LONG = 4096;
         constexpr int NT2 = W == 1 ? 512 : 1024;
-        const bool stage2 = W == 1 && !(c->opts.flags & UC_FLAG_DIRECT_SCATTER) &&
-                            sub_lds_bytes<W>(round2, s1max, keep_src, true, NT2 / 64) <= c->lds_limit;
+        const bool want_stage = !(c->opts.flags & UC_FLAG_DIRECT_SCATTER);
+        auto fits = [&](uint32_t round, bool stage) {
+            return sub_lds_bytes<W>(round, s1max, keep_src, stage, NT2 / 64) <= c->lds_limit;
+        };
+        const bool stage2 = want_stage && fits(R_SHORT, true);
+        const uint32_t round2 = stage2 && c->m / GR >= LONG_ROW && fits(R_LONG, true) ? R_LONG : R_SHORT;
+        const uint32_t tile2 = SUB_TILE;
         c->tile2 = tile2;
         // tiles: at most one partial tile per row beyond m / tile2
         const uint64_t T2 = GR + (c->m + tile2 - 1) / tile2;
@@ -4589,18 +4590,19 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         CHK(ensure(c, c->flags, c->m + 64));
         if (keep_src) CHK(ensure(c, c->src, c->m * 4));
         CHK(ensure(c, c->perm, c->m * 4));
-#define UC_S2(ST)                                                                                                   \
+#define UC_S2(ST, ROUND)                                                                                           \
     do {                                                                                                           \
-        const size_t lds2 = sub_lds_bytes<W>(round2, s1max, keep_src, ST, NT2 / 64);                                 \
-        CHK(allow_lds(c, k_sub_scatter<W, ST, IPT2 * BLOCK / NT2, NT2>, lds2));                                    \
-        KLAUNCH(c, "k_sub_scatter", (k_sub_scatter<W, ST, IPT2 * BLOCK / NT2, NT2>), (xcd_grid(T2), NT2, lds2),      \
+        const size_t lds2 = sub_lds_bytes<W>(ROUND, s1max, keep_src, ST, NT2 / 64);                                 \
+        CHK(allow_lds(c, k_sub_scatter<W, ST, ROUND / NT2, NT2>, lds2));                                           \
+        KLAUNCH(c, "k_sub_scatter", (k_sub_scatter<W, ST, ROUND / NT2, NT2>), (xcd_grid(T2), NT2, lds2),             \
                 P<BTile>(c->tiles2), P<uint16_t>(c->sub), P<uint32_t>(c->hist2), P<uint32_t>(c->fboff),             \
-                row_first, P<uint64_t>(c->kmer2), keep_src ? P<uint32_t>(c->src2) : nullptr,          \
-                P<uint64_t>(c->kmer), P<uint8_t>(c->flags), keep_src ? P<uint32_t>(c->src) : nullptr,               \
-                P<uint32_t>(c->perm), tile_arg_xcd(T2));                                                           \
+                row_first, P<uint64_t>(c->kmer2), keep_src ? P<uint32_t>(c->src2) : nullptr, P<uint64_t>(c->kmer),  \
+                P<uint8_t>(c->flags), keep_src ? P<uint32_t>(c->src) : nullptr, P<uint32_t>(c->perm),               \
+                tile_arg_xcd(T2));                                                                                 \
     } while (0)
-        if (stage2) UC_S2(true);
-        else UC_S2(false);
+        if (round2 == R_LONG) UC_S2(true, R_LONG);
+        else if (stage2) UC_S2(true, R_SHORT);
+        else UC_S2(false, R_SHORT);
 #undef UC_S2
         if (c->x)
             KLAUNCH(c, "k_pair_remap", k_pair_remap, (grid_for(c->x, PAIR_ITEMS * BLOCK), BLOCK, 0), P<uint32_t>(c->pair_h),
