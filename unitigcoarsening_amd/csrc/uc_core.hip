@@ -2490,10 +2490,12 @@ __global__ void k_chain_tail(const uint32_t *__restrict__ list, const uint32_t *
 // Chain ranking, unitig lengths and the totals of a small job in one workgroup
 // (the same steps as k_chain_init, SPEC_ROUNDS of k_chain_round, k_chain_tail
 // and the scans of the tile sums, which are four to ten launches of 3-5 us
-// each with next to nothing in them): up to CHAIN_ONE_TILES tiles, and as many
-// sampled splitters as its threads can stride over.
+// each with next to nothing in them): up to CHAIN_ONE_TILES tiles (their sums
+// fill LDS; jobs of 3-8 M slots gain 2-5% of their step over the launches, which
+// a graph had replayed), and as many sampled splitters as its threads can stride
+// over.
 constexpr int CHAIN_ONE_NT = 1024;
-constexpr uint32_t CHAIN_ONE_TILES = 6144, CHAIN_ONE_LIST = 16384;
+constexpr uint32_t CHAIN_ONE_TILES = 18432, CHAIN_ONE_LIST = 20480;
 
 __global__ __launch_bounds__(CHAIN_ONE_NT) void k_chain_one(const uint32_t *__restrict__ list, uint32_t *cnt,
                                                             const uint32_t *__restrict__ hasp,
@@ -5088,6 +5090,7 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
     auto spec_pass = [&]() -> int {
         CHK(walks());
         if (one) {
+            CHK(allow_lds(c, k_chain_one, T * 8 + 1024));
             KLAUNCH(c, "k_chain_one", k_chain_one, (1, CHAIN_ONE_NT, T * 8), P<uint32_t>(c->list), cnt,
                     P<uint32_t>(c->hasp), P<uint32_t>(c->prevseg), P<uint64_t>(c->seg), ca, cb, P<uint32_t>(c->ulen),
                     P<uint64_t>(c->tsum), P<uint64_t>(c->tcnt), (uint32_t)T, ct);
