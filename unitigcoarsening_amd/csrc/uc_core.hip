@@ -2212,33 +2212,43 @@ __host__ __device__ constexpr uint32_t ct_tile(uint64_t m)
     return t;
 }
 
-// the borrowed duplicate's out-edge moves to the home copy; the target keeps
-// its has-predecessor bit
+// The borrowed duplicate's out-edge moves to the home copy's run: a lent k-mer
+// ends its run, and the run continues through the duplicate's edge (the target
+// keeps its has-predecessor bit).  Records end without a next run, so only real
+// edges are written.  Contraction follows records; the home copies' own links
+// still hold their run heads and are spliced when something reads links
+// (k_splice_links): the fourth random access per pair took a quarter of the
+// kernel.
 __global__ __launch_bounds__(BLOCK) void k_splice(const uint32_t *__restrict__ pair_home,
                                                   const uint32_t *__restrict__ pair_borrow, uint32_t x,
-                                                  uint32_t *__restrict__ link, uint64_t *__restrict__ rec)
+                                                  const uint32_t *__restrict__ link, uint64_t *__restrict__ rec)
 {
     const uint32_t i0 = blockIdx.x * (PAIR_ITEMS * BLOCK) + threadIdx.x;
     if (i0 >= x) return;
-    uint32_t h[PAIR_ITEMS], l[PAIR_ITEMS], head[PAIR_ITEMS];
+    uint32_t l[PAIR_ITEMS], head[PAIR_ITEMS];
 #pragma unroll
     for (int j = 0; j < PAIR_ITEMS; j++) {  // (past the end: the first pair again)
         const uint32_t i = i0 + (uint32_t)j * BLOCK, c = i < x ? i : i0;
-        h[j] = pair_home[c];
+        head[j] = pair_home[c];
         l[j] = pair_borrow[c];
     }
 #pragma unroll
     for (int j = 0; j < PAIR_ITEMS; j++) {
         l[j] = link[l[j]];
-        head[j] = link[h[j]];  // the lent k-mer's run head
+        head[j] = link[head[j]];  // the lent k-mer's run head
     }
 #pragma unroll
-    for (int j = 0; j < PAIR_ITEMS; j++) {
-        if (i0 + (uint32_t)j * BLOCK >= x) continue;
-        link[h[j]] = l[j];
-        // a lent k-mer ends its run: the run continues through the duplicate's edge
-        reinterpret_cast<uint32_t *>(rec)[2ull * head[j]] = l[j];  // the record's next-run field
-    }
+    for (int j = 0; j < PAIR_ITEMS; j++)
+        if (i0 + (uint32_t)j * BLOCK < x && l[j] != NONE)
+            reinterpret_cast<uint32_t *>(rec)[2ull * head[j]] = l[j];  // the record's next-run field
+}
+
+// the same for the home copies' links (successors from here on, not run heads)
+__global__ void k_splice_links(const uint32_t *__restrict__ pair_home, const uint32_t *__restrict__ pair_borrow,
+                               uint32_t x, uint32_t *__restrict__ link)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < x) link[pair_home[i]] = link[pair_borrow[i]];
 }
 
 // list index for every flagged lane: one atomic per wave
@@ -3240,7 +3250,8 @@ struct uc_ctx {
     std::vector<uint32_t> cb_first;  // first fine bucket of every coarse bucket
     std::vector<uint32_t> fboff_h;   // fine bucket rows
     bool loaded = false, bucketed = false, edged = false, coarsened = false, emitted = false;
-    bool spliced = false;  // lent k-mers' links hold successors, no longer run heads
+    bool spliced = false;  // the runs of lent k-mers continue through their duplicates' edges
+    bool links_spliced = false;  // and their own links hold successors, no longer run heads
     bool edges_ready = false;
     std::vector<uint64_t> et_toff, et_first;
     std::vector<uint32_t> et_cap;
@@ -5209,6 +5220,17 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
     return UC_OK;
 }
 
+// lent k-mers' links after the splice, for what reads links
+int splice_links(uc_ctx *c)
+{
+    if (c->links_spliced) return UC_OK;
+    if (c->x)
+        KLAUNCH(c, "k_splice_links", k_splice_links, (grid_for(c->x), BLOCK, 0), P<uint32_t>(c->pair_h),
+                P<uint32_t>(c->pair_b), (uint32_t)c->x, P<uint32_t>(c->link));
+    c->links_spliced = true;
+    return UC_OK;
+}
+
 // isolated cycles: every k-mer no head reaches lies on one; each cycle is
 // cut in front of its lexicographically smallest k-mer
 template <int W>
@@ -5216,6 +5238,7 @@ int cut_cycles(uc_ctx *c, uint64_t *n_cut)
 {
     const uint32_t m = (uint32_t)c->m;
     uint32_t *cnt = P<uint32_t>(c->small);
+    CHK(splice_links(c));
     KLAUNCH(c, "k_cover", k_cover, (grid_for(m), BLOCK, 0), P<uint64_t>(c->rec), P<uint32_t>(c->hasp),
             P<uint8_t>(c->flags), c->chain, m, c->salt, c->shift);
     CHK(fill<uint32_t>(c, cnt + C_CYC, 1, 0u));
@@ -5297,6 +5320,7 @@ int do_coarsen(uc_ctx *c, bool defer)
         KLAUNCH(c, "k_splice", k_splice, (grid_for(c->x, PAIR_ITEMS * BLOCK), BLOCK, 0), P<uint32_t>(c->pair_h), P<uint32_t>(c->pair_b),
                 (uint32_t)c->x, P<uint32_t>(c->link), P<uint64_t>(c->rec));
     }
+    if (!c->spliced) c->links_spliced = false;
     c->spliced = true;
     uint64_t live = 0;
     uint32_t nonconv = 0;
@@ -5896,6 +5920,7 @@ int uc_succ_copy(uc_ctx *c, uint32_t *succ)
     if (!c->edged) return fail(c, UC_E_STATE, "no edge result");
     CHK(select_dev(c));
     CHK(ensure(c, c->hit, c->m * 4));  // (UC_FLAG_LOW_MEMORY frees it after the edge phase)
+    if (c->spliced) CHK(splice_links(c));
     if (c->m) KLAUNCH(c, "k_link_succ", k_link_succ, (std::min<uint32_t>(grid_for(c->m), 65536), BLOCK, 0),
                       P<uint32_t>(c->link), P<uint8_t>(c->flags), (uint32_t)c->m, !c->spliced, P<uint32_t>(c->hit));
     return d2h(c, succ, c->hit.p, c->m * 4);
