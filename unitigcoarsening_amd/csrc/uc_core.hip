@@ -1888,20 +1888,23 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
     // inside: the occupant's k-mer is read whether or not there is one (any
     // staged slot does for an empty entry).  A CU has one scalar unit, and the
     // masks of nested branches kept it busier than the vector units (323 M
-    // scalar against 268 M vector instructions on the 50 Mbp job).  A table
-    // holds at most half as many keys as entries, so every probe ends.
+    // scalar against 268 M vector instructions on the 50 Mbp job).  A
+    // round lasts as long as its slowest lane, so probes go by growing steps,
+    // which keep clusters short (edge phase 613 -> 580 us against the next
+    // entry); they reach every entry of a power of two, and a table holds at
+    // most half as many keys as entries, so every probe ends.
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
         if (hpos[e] == NONE) continue;
         const uint32_t i = threadIdx.x + (uint32_t)e * EB;
         const Kmer<W> key = prefix_key<W>(xs[e], pm0, pm1);
-        uint32_t pos = hpos[e], at, cur, more;
+        uint32_t pos = hpos[e], step = 0, at, cur, more;
         do {
             if (CNT) np++;
             at = pos;
             cur = atomicCAS(&tab[at], LDS_EMPTY, i);
             more = min(cur + 1u, prefix_diff<W>(km[min(cur & 0xFFFFu, last)], key, pm0, pm1));
-            pos = (pos + 1) & tmask;
+            pos = (pos + ++step) & tmask;
         } while (more);  // neither empty (cur + 1 = 0) nor the same key
         opaque(cur);
         if (cur != LDS_EMPTY) atomicOr(&tab[at], LDS_SHARED);
@@ -1919,13 +1922,13 @@ __global__ __launch_bounds__(EB) void k_edge_lds(const uint64_t *__restrict__ km
         uint16_t hp = LDS_NOHIT;
         if (hpos[e] != NONE) {
             const Kmer<W> key = suffix_key<W>(xs[e]);
-            uint32_t pos = hpos[e], at, en, more;
+            uint32_t pos = hpos[e], step = 0, at, en, more;
             do {
                 if (CNT) np++;
                 at = pos;
                 en = tab[at];
                 more = min(en + 1u, prefix_diff<W>(km[min(en & 0xFFFFu, last)], key, pm0, pm1));
-                pos = (pos + 1) & tmask;
+                pos = (pos + ++step) & tmask;
             } while (more);
             opaque(en);
             if (en != LDS_EMPTY) {
