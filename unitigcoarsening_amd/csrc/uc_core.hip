@@ -1054,6 +1054,7 @@ __global__ void k_gather_boff(const uint32_t *__restrict__ hscan, const uint64_t
 
 // one workgroup: tiles and histogram entries per coarse bucket, prefixes
 constexpr int PLAN_NT = 1024;  // one workgroup walks all coarse buckets: the widest one
+constexpr uint32_t PLAN_ROWS = 4;
 
 __global__ __launch_bounds__(PLAN_NT) void k_plan2_prefix(const uint32_t *__restrict__ boff,
                                                         const uint32_t *__restrict__ cb_first, uint32_t G, uint32_t tile,
@@ -1065,13 +1066,23 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan2_prefix(const uint32_t *__rest
     if (threadIdx.x == 0) tcarry = hcarry = 0;
     __syncthreads();
     const int w = threadIdx.x / 64;
-    for (uint32_t g0 = 0; g0 < G; g0 += PLAN_NT) {
-        const uint32_t g = g0 + threadIdx.x;
+    // (PLAN_ROWS rows per thread: a round's barriers and scans cost the same
+    // whatever the rows; 256 sets: 45 -> 25 us)
+    for (uint32_t g0 = 0; g0 < G; g0 += PLAN_NT * PLAN_ROWS) {
+        const uint32_t g = g0 + threadIdx.x * PLAN_ROWS;
+        uint32_t b[PLAN_ROWS + 1], f[PLAN_ROWS + 1];
+#pragma unroll
+        for (uint32_t i = 0; i <= PLAN_ROWS; i++) {
+            b[i] = boff[min(g + i, G)];
+            f[i] = cb_first[min(g + i, G)];
+        }
         uint64_t ts = 0, hs = 0;
-        if (g < G) {
-            const uint32_t rows = boff[g + 1] - boff[g];
-            ts = rows ? (rows + tile - 1) / tile : 1u;
-            hs = ts * (cb_first[g + 1] - cb_first[g]);
+#pragma unroll
+        for (uint32_t i = 0; i < PLAN_ROWS; i++) {
+            const uint32_t rows = b[i + 1] - b[i];
+            b[i] = g + i < G ? (rows ? (rows + tile - 1) / tile : 1u) : 0u;
+            ts += b[i];
+            hs += (uint64_t)b[i] * (f[i + 1] - f[i]);
         }
         const uint64_t ti = wave_incl_scan(ts), hi = wave_incl_scan(hs);
         if (__lane_id() == 63) {
@@ -1088,10 +1099,15 @@ __global__ __launch_bounds__(PLAN_NT) void k_plan2_prefix(const uint32_t *__rest
             tt += wsum[q];
             ht += hsum[q];
         }
-        if (g < G) {
-            cb_ts[g] = (uint32_t)ts;
-            cb_tfirst[g] = (uint32_t)tp;
-            cb_hbase[g] = hp;
+#pragma unroll
+        for (uint32_t i = 0; i < PLAN_ROWS; i++) {
+            if (g + i < G) {
+                cb_ts[g + i] = b[i];
+                cb_tfirst[g + i] = (uint32_t)tp;
+                cb_hbase[g + i] = hp;
+            }
+            tp += b[i];
+            hp += (uint64_t)b[i] * (f[i + 1] - f[i]);
         }
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -1694,26 +1710,37 @@ constexpr uint32_t PLAN_RUN = 8;  // fine buckets per planning thread
 constexpr uint32_t GROUPS_WANTED = 512, GROUP_PACK_MIN = 256;
 static_assert(MAX_SUB <= PLAN_RUN * BLOCK, "one run of fine buckets per planning thread");
 
-__device__ __forceinline__ uint32_t pack_groups(const uint32_t *__restrict__ fboff, uint32_t f0, uint32_t v0,
-                                                uint32_t v1, uint32_t gpack, uint32_t gmax, EGroup *out,
-                                                uint32_t *__restrict__ over, uint32_t *__restrict__ n_over)
+// The row starts of fine buckets [v0, v1) (at most PLAN_RUN, from f0 on) and the
+// last one's end, all loads in flight at once; buckets past v1 read as empty,
+// which open no group.  (Read one by one in the packing loop they were a chain
+// of eight loads per pass.)
+struct PlanRows {
+    uint32_t r[PLAN_RUN + 1];
+};
+__device__ __forceinline__ PlanRows plan_rows(const uint32_t *__restrict__ fboff, uint32_t f0, uint32_t v0, uint32_t v1)
+{
+    PlanRows x;
+#pragma unroll
+    for (uint32_t i = 0; i <= PLAN_RUN; i++) x.r[i] = fboff[f0 + min(v0 + i, v1)];
+    return x;
+}
+
+__device__ __forceinline__ uint32_t pack_groups(const PlanRows &x, uint32_t first, uint32_t gpack, uint32_t gmax,
+                                                EGroup *out, uint32_t *__restrict__ over, uint32_t *__restrict__ n_over)
 {
     uint32_t ng = 0, gb = 0, ge = 0;
     bool open = false;
-    for (uint32_t v = v0; v < v1; v++) {
-        const uint32_t r0 = fboff[f0 + v], r1 = fboff[f0 + v + 1];
+#pragma unroll
+    for (uint32_t i = 0; i < PLAN_RUN; i++) {
+        const uint32_t r0 = x.r[i], r1 = x.r[i + 1];
         if (r1 - r0 > gmax) {
-            if (over) over[atomicAdd(n_over, 1u)] = f0 + v;
+            if (over) over[atomicAdd(n_over, 1u)] = first + i;
             if (open && out) out[ng] = EGroup{gb, ge};
             ng += open;
             open = false;
-            continue;
-        }
-        if (open && r1 - gb <= gpack) {
+        } else if (open && r1 - gb <= gpack) {
             ge = r1;
-        } else if (r1 == r0) {
-            continue;  // an empty fine bucket opens no group
-        } else {
+        } else if (r1 != r0) {  // (an empty fine bucket opens no group)
             if (open && out) out[ng] = EGroup{gb, ge};
             ng += open;
             gb = r0;
@@ -1725,8 +1752,12 @@ __device__ __forceinline__ uint32_t pack_groups(const uint32_t *__restrict__ fbo
     return ng + open;
 }
 
-// per coarse bucket: its group count (block sum of the threads' counts)
-__global__ __launch_bounds__(BLOCK) void k_plan_count(const uint32_t *__restrict__ fboff,
+// per coarse bucket: its group count (the sum of the threads' counts).  One wave
+// where every coarse bucket's runs fit its lanes (256 sets: 16384 coarse buckets
+// of one or two runs: count 25.5 and write 25.7 us in four waves with their loads
+// one by one, 7.7 and 8.7 so), else four.
+template <int NT>
+__global__ __launch_bounds__(NT) void k_plan_count(const uint32_t *__restrict__ fboff,
                                                       const uint32_t *__restrict__ cb_first, uint32_t gpack,
                                                       uint32_t gmax, uint32_t *__restrict__ gcount, uint32_t *__restrict__ over,
                                                       uint32_t *__restrict__ n_over)
@@ -1734,16 +1765,23 @@ __global__ __launch_bounds__(BLOCK) void k_plan_count(const uint32_t *__restrict
     __shared__ uint32_t red[WAVES];
     const uint32_t g = blockIdx.x, f0 = cb_first[g], S = cb_first[g + 1] - f0;
     // S <= MAX_SUB <= PLAN_RUN * BLOCK: one run of fine buckets per thread
-    const uint32_t v0 = PLAN_RUN * threadIdx.x, v1 = v0 + PLAN_RUN < S ? v0 + PLAN_RUN : S;
-    const uint32_t ng = v0 < S ? pack_groups(fboff, f0, v0, v1, gpack, gmax, nullptr, over, n_over) : 0u;
-    const uint32_t tot = block_reduce(ng, red);
-    if (threadIdx.x == 0) gcount[g] = tot;
+    const uint32_t v0 = min(PLAN_RUN * threadIdx.x, S), v1 = min(v0 + PLAN_RUN, S);
+    const PlanRows x = plan_rows(fboff, f0, v0, v1);
+    const uint32_t ng = pack_groups(x, f0 + v0, gpack, gmax, nullptr, over, n_over);
+    if constexpr (NT == 64) {
+        const uint32_t incl = wave_incl_scan(ng);
+        if (threadIdx.x == 63) gcount[g] = incl;
+    } else {
+        const uint32_t tot = block_reduce(ng, red);
+        if (threadIdx.x == 0) gcount[g] = tot;
+    }
 }
 
 // per coarse bucket: its groups from its scanned first entry
 // (and, when given, a copy of two counters beside the offsets, for the same
 // host read)
-__global__ __launch_bounds__(BLOCK) void k_plan_write(const uint32_t *__restrict__ fboff,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_plan_write(const uint32_t *__restrict__ fboff,
                                                       const uint32_t *__restrict__ cb_first, uint32_t gpack,
                                                       uint32_t gmax, const uint32_t *__restrict__ gfirst,
                                                       EGroup *__restrict__ groups, const uint32_t *__restrict__ tot,
@@ -1752,15 +1790,18 @@ __global__ __launch_bounds__(BLOCK) void k_plan_write(const uint32_t *__restrict
     __shared__ uint32_t wsum[WAVES];
     if (tot && blockIdx.x == 0 && threadIdx.x < 2) tot_out[threadIdx.x] = tot[threadIdx.x];
     const uint32_t g = blockIdx.x, f0 = cb_first[g], S = cb_first[g + 1] - f0;
-    const uint32_t v0 = PLAN_RUN * threadIdx.x, v1 = v0 + PLAN_RUN < S ? v0 + PLAN_RUN : S;
-    const uint32_t ng = v0 < S ? pack_groups(fboff, f0, v0, v1, gpack, gmax, nullptr, nullptr, nullptr) : 0u;
+    const uint32_t v0 = min(PLAN_RUN * threadIdx.x, S), v1 = min(v0 + PLAN_RUN, S);
+    const PlanRows x = plan_rows(fboff, f0, v0, v1);
+    const uint32_t ng = pack_groups(x, f0 + v0, gpack, gmax, nullptr, nullptr, nullptr);
     const uint32_t incl = wave_incl_scan(ng);
-    const int w = threadIdx.x / 64;
-    if (__lane_id() == 63) wsum[w] = incl;
-    __syncthreads();
     uint32_t base = gfirst[g] + incl - ng;
-    for (int q = 0; q < w; q++) base += wsum[q];
-    if (ng) pack_groups(fboff, f0, v0, v1, gpack, gmax, groups + base, nullptr, nullptr);
+    if constexpr (NT > 64) {
+        const int w = threadIdx.x / 64;
+        if (__lane_id() == 63) wsum[w] = incl;
+        __syncthreads();
+        for (int q = 0; q < w; q++) base += wsum[q];
+    }
+    if (ng) pack_groups(x, f0 + v0, gpack, gmax, groups + base, nullptr, nullptr);
 }
 
 // The whole plan of a small job of one set in one workgroup, a thread per run
@@ -1780,8 +1821,9 @@ __global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__rest
     __syncthreads();
     const uint32_t rp = (S + PLAN_RUN - 1) / PLAN_RUN;  // runs per coarse bucket
     const uint32_t g = threadIdx.x / rp, j = threadIdx.x % rp;
-    const uint32_t v0 = j * PLAN_RUN, v1 = min(S, v0 + PLAN_RUN);
-    const uint32_t ng = g < G ? pack_groups(fboff, g * S, v0, v1, gpack, gmax, nullptr, over, &n_over) : 0u;
+    const uint32_t f0 = min(g, G - 1) * S, v0 = g < G ? j * PLAN_RUN : S, v1 = min(S, v0 + PLAN_RUN);
+    const PlanRows x = plan_rows(fboff, f0, v0, v1);
+    const uint32_t ng = pack_groups(x, f0 + v0, gpack, gmax, nullptr, over, &n_over);
     const uint32_t incl = wave_incl_scan(ng);
     const int w = threadIdx.x / 64;
     if (__lane_id() == 63) wsum[w] = incl;
@@ -1792,7 +1834,7 @@ __global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__rest
         all += wsum[q];
     }
     if (g < G && j == 0) gfirst[g] = base;
-    if (ng) pack_groups(fboff, g * S, v0, v1, gpack, gmax, groups + base, nullptr, nullptr);
+    if (ng) pack_groups(x, f0 + v0, gpack, gmax, groups + base, nullptr, nullptr);
     if (threadIdx.x == 0) {
         gfirst[G] = all;
         gfirst[G + 1] = n_over;
@@ -4849,13 +4891,17 @@ int prepare_edges(uc_ctx *c)
                     group_pack, group_max, gfd, P<EGroup>(c->egroups), P<uint32_t>(c->over), pend ? cnt + C_TOT : nullptr);
         } else {
             CHK(fill<uint32_t>(c, gfd + G + 1, 1, 0u));
-            KLAUNCH(c, "k_plan_count", k_plan_count, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->fboff),
-                    P<uint32_t>(c->cbfirst), group_pack, group_max, gfd, P<uint32_t>(c->over), gfd + G + 1);
+            const uint32_t smax = *std::max_element(c->set_sub.begin(), c->set_sub.end());
+            const bool wave = smax <= 64 * PLAN_RUN;
+            const uint32_t nt = wave ? 64 : BLOCK;
+            KLAUNCH(c, "k_plan_count", (wave ? k_plan_count<64> : k_plan_count<BLOCK>), ((uint32_t)G, nt, 0),
+                    P<uint32_t>(c->fboff), P<uint32_t>(c->cbfirst), group_pack, group_max, gfd, P<uint32_t>(c->over),
+                    gfd + G + 1);
             CHK(scan_excl<uint32_t>(c, gfd, gfd, G, gfd + G, c->scan_tmp));
             // (sizes the bucketing left on the device come along: placements, crossings)
-            KLAUNCH(c, "k_plan_write", k_plan_write, ((uint32_t)G, BLOCK, 0), P<uint32_t>(c->fboff),
-                    P<uint32_t>(c->cbfirst), group_pack, group_max, gfd, P<EGroup>(c->egroups), pend ? cnt + C_TOT : nullptr,
-                    gfd + G + 2);
+            KLAUNCH(c, "k_plan_write", (wave ? k_plan_write<64> : k_plan_write<BLOCK>), ((uint32_t)G, nt, 0),
+                    P<uint32_t>(c->fboff), P<uint32_t>(c->cbfirst), group_pack, group_max, gfd, P<EGroup>(c->egroups),
+                    pend ? cnt + C_TOT : nullptr, gfd + G + 2);
         }
         gf.resize(G + 4);
         CHK(d2h(c, gf.data(), gfd, (G + (pend ? 4 : 2)) * 4));
