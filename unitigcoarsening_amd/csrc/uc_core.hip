@@ -3,23 +3,24 @@
 // Pipeline of one job (reference phases in brackets):
 //   1. bucketing   [lmin_buckets.h:288-433, driver.cpp:137-225]
 //      k_lmin_count: prefix/suffix l-minimizers per k-mer, per-tile bucket
-//      histogram in LDS; device scan; k_lmin_scatter: stable wavefront-
-//      ballot ranking, LDS-staged coalesced writes, crossing k-mers
-//      duplicated into their suffix bucket, (home, borrow) pair list;
-//      k_sub_count / k_sub_scatter: the same counting sort of each coarse
-//      bucket by the next bits of the minimizer order (fine buckets).
+//      histogram in LDS; device scan; k_lmin_scatter: stable ranks by
+//      bitwise match over the wave, LDS-staged coalesced writes, crossing
+//      k-mers duplicated into their suffix bucket, (home, borrow) pair list;
+//      k_sub_count / k_sub_scatter: the same counting sort of each pass-1
+//      row by the remaining bits of the minimizer order (fine buckets).
 //   2. edge finding [assembler.h:113-214]
 //      k_edge_lds: one workgroup per group of fine buckets, k-mers staged
 //      in LDS, insert / lookup / resolve against an LDS table; edges inside
-//      the group are chained into runs by pointer jumping in LDS.  Fine
-//      buckets too large for LDS use HBM tables (k_edge_insert / lookup /
-//      resolve).
+//      the group are followed into runs from their heads in LDS.  Larger
+//      fine buckets are split by key hash (k_edge_slice), the largest use HBM
+//      tables (k_edge_insert / lookup / resolve).
 //   3. contraction [coarseners.h:68-485, heuristics.h:105-256,
 //      compact_graph.h, driver.cpp:527-587]
 //      k_splice re-attaches each borrowed duplicate's out-edge to its home
-//      copy; splitters (path heads + a hashed 2^-s sample of run heads)
+//      copy's run record; splitters (path heads + a hashed 2^-s sample of run heads)
 //      walk their segment run by run (k_seg_count); segment chains are
-//      ranked by pointer jumping (k_chain_*).  Isolated cycles are cut at
+//      ranked by pointer jumping (k_chain_one in one workgroup, k_chain_* over
+//      the chip for the largest jobs).  Isolated cycles are cut at
 //      their lexicographically smallest k-mer and the contraction repeats.
 //   4. emission    [compact.h:59-210, lmin_buckets.h:172-283]
 //      k_head_emit / k_rand_emit write each unitig: its first k-mer, then
@@ -540,9 +541,11 @@ __device__ __forceinline__ uint2 get_codes(const void *__restrict__ bkt, uint64_
 
 // Pass 1 sorts by the coarse bucket and the top J bits of the fine index
 // (rows of pass 1: B << J per set); pass 2 sorts each row by the remaining s1
-// bits.  A pass's counters, ballots and piece lengths go with its own bucket
-// count (50 Mbp job, 64 x 512 buckets, the two scatters: 6 + 9 bits 529 + 515 us,
-// 7 + 8 bits 553 + 448, 8 + 7 bits 615 + 387).
+// bits.  A pass's counters, match steps and piece lengths go with its own bucket
+// count (50 Mbp job, 64 x 512 buckets, the two scatters when ranks were ballots
+// per bit: 6 + 9 bits 529 + 515 us, 7 + 8 bits 553 + 448, 8 + 7 bits 615 + 387;
+// with the ranks in registers 7 + 8 bits take 300 + 367, and a bit more in pass 1
+// makes the whole job 3% slower).
 // A k-mer's code is its fine bucket in slot order: coarse bucket above, fine
 // index below, the fine index of a set with fewer than J fine bits moved up
 // (the rows between stay empty), so row = code >> s1 and equal codes are equal
@@ -762,8 +765,10 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t *a, uint32_t n, uin
 // Stable scatter into the bucket CSR: inside a tile, placements keep the
 // order of their k-mers (home copy before borrowed copy when both land in
 // one bucket); per wave the rank among placements bound for the same bucket
-// comes from log2(B) ballots of the bucket bits.  Every thread's codes and
-// k-mers are loaded up front, so all of them are in flight at once.  With
+// comes from matching the bucket number bit by bit (match_bit).  Every thread's
+// codes and k-mers are loaded up front, so all of them are in flight at once.
+// (48 M 31-mers: 550 us with an array of lane masks per bit, 300 so; 226
+// instructions per k-mer, 276 us of them, bound it, not its 1.2 GB.)  With
 // STAGE, the tile's placements are gathered in LDS in bucket order and leave
 // as runs of consecutive slots; a tile with more placements than the stage
 // holds (more than a quarter of its k-mers crossing) stores them directly.
@@ -1244,12 +1249,14 @@ __global__ __launch_bounds__(BLOCK) void k_sub_rows(const uint32_t *__restrict__
 
 // Pass-2 scatter with LDS staging.  A planned tile (up to SUB_TILE slots of one
 // coarse bucket, in rounds of IPT * NT) is sorted round by round; each round is
-// ranked per wave: each wave owns a chunk of consecutive slots, counts its
-// slots per fine bucket (ballot groups, one LDS add per group), the counts are
-// scanned once per round, and a second sweep gives every slot its stable
+// ranked per wave: each wave owns a chunk of consecutive slots, matches their
+// fine buckets bit by bit (match_bit; one LDS add per bucket met), the counts
+// are scanned once per round, and a second sweep gives every slot its stable
 // position inside the round, sorted by fine bucket.  The slots are staged
 // there in LDS and written out in that order, so consecutive lanes store
-// consecutive addresses of one fine bucket's run.  The running base of every
+// consecutive addresses of one fine bucket's run: the pieces are a few dozen
+// bytes, and their half-written lines bound it (50 Mbp job: 520 -> 367 us for
+// 1.37 GB, 3.7 TB/s).  The running base of every
 // fine bucket carries from round to round, so the histogram holds one row per
 // planned tile (not one per round), and the next round's
 // slots are loaded while the current one is ranked.
@@ -1356,7 +1363,7 @@ __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ ti
             gbase[v] += b - t0;
         }
         __syncthreads();
-        // 3. stable positions: per pass, ballot groups of equal fine index
+        // 3. stable positions: per pass, matched groups of equal fine index
 #pragma unroll
         for (int j = 0; j < IPT; j++) {
             const bool valid = vf[j] != NONE;
@@ -1416,6 +1423,8 @@ __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ ti
 
 // (the pair count is *xdev when given: the host has not read it, and x is
 // then its bound)
+// (random lines bound it: 50 Mbp job, 4.6 M pairs, 90 us, whatever the pairs per
+// thread; 7 M k-mers, with the splice, 8 us less than a pair per thread)
 constexpr int PAIR_ITEMS = 4;  // pairs per thread: their random reads are in flight together
 
 __global__ __launch_bounds__(BLOCK) void k_pair_remap(uint32_t *__restrict__ pair_home, uint32_t *__restrict__ pair_borrow,
@@ -1851,7 +1860,9 @@ __global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__rest
 // Keys of different fine buckets never match (equal (k-1)-mers have
 // equal minimizers), so a group shares one table.  HBM sees only the
 // sequential k-mer/flag reads and link writes plus one bitmap word per 32
-// slots.
+// slots.  Instructions bound it (50 Mbp job: 321 per slot, 431 of its 499 us,
+// 790 before the probe loops had one exit, the hash one multiply fewer and the
+// hits stayed in registers); its 1.0 GB would take 220 us.
 //   LDS layout (nb = launch capacity, a power of two):
 //     km   Kmer<W>[nb]   staged k-mers
 //     tab  uint32[2nb]   owner (16 bits) | LDS_SHARED | hits << 24, or LDS_EMPTY
@@ -2272,7 +2283,7 @@ __host__ __device__ constexpr uint32_t ct_tile(uint64_t m)
 // edges are written.  Contraction follows records; the home copies' own links
 // still hold their run heads and are spliced when something reads links
 // (k_splice_links): the fourth random access per pair took a quarter of the
-// kernel.
+// kernel (50 Mbp job: 210 -> 152 us, all random lines).
 __global__ __launch_bounds__(BLOCK) void k_splice(const uint32_t *__restrict__ pair_home,
                                                   const uint32_t *__restrict__ pair_borrow, uint32_t x,
                                                   const uint32_t *__restrict__ link, uint64_t *__restrict__ rec)
@@ -2367,7 +2378,8 @@ __device__ __forceinline__ uint64_t mlist_entry(uint32_t off, bool multi, uint32
 // the splitters that walk on (5% of the slots) are gathered first, so that one
 // thread takes one walk and all of a tile's chains of random reads are in
 // flight at once (with each thread walking its own slots one after another a
-// wave followed 2-3 walks at a time, eight times).
+// wave followed 2-3 walks at a time, eight times).  50 Mbp job: 310 -> 147 us,
+// bound by the latency of the walks' reads.
 template <int CT>
 __global__ __launch_bounds__(CT_NT) void k_seg_count(const uint64_t *__restrict__ rec, const uint32_t *__restrict__ hasp,
                                                      const uint8_t *__restrict__ flags, uint32_t m, uint32_t salt,
@@ -2901,8 +2913,8 @@ constexpr uint32_t emit_stage() { return W == 1 ? 2560 : 4608; }
 
 // Per tile: the live heads are gathered in slot order (39% of the slots:
 // walking the slots themselves left 61% of every wave's lanes idle through the
-// spelling, 0.85 ms on the 50 Mbp job), a scan of their lengths gives their
-// text offsets, and the wave takes 64 of them at a time: one contiguous text
+// spelling, 0.85 ms on the 50 Mbp job, 0.51 so: 2.45 GB at 4.7 TB/s, what a
+// copy reaches), a scan of their lengths gives their text offsets, and the wave takes 64 of them at a time: one contiguous text
 // range, spelled into its LDS stage (put_kmer_lds, put_rest) and
 // written as aligned 16-byte lines, or straight to HBM when it does not fit.
 // A thread's next head (record and k-mer) is loaded while it writes the
