@@ -71,8 +71,8 @@ def kernel_bytes(name, n, m, x, W, n_unitigs, text_bytes, k, runs):
         "k_edge_lookup": m * (1 + kb + 4) + (m - x) * (16 + kb),
         "k_edge_resolve": m * (4 + 8) + (m - x) * 16 + m // 8,
         # pair entries, the duplicate's link, the lent k-mer's link (its run
-        # head); write that link and its run record's next run
-        "k_splice": x * (4 + 4 + 4 + 4 + 4 + 4),
+        # head); write its run record's next run
+        "k_splice": x * (4 + 4 + 4 + 4 + 4),
         # read flag + has-predecessor bit per slot, one run record per run
         # (the list entries of heads of several runs are not counted)
         "k_seg_count": m * 1 + m // 8 + runs * 8,

@@ -1255,8 +1255,8 @@ __global__ __launch_bounds__(BLOCK) void k_sub_rows(const uint32_t *__restrict__
 // position inside the round, sorted by fine bucket.  The slots are staged
 // there in LDS and written out in that order, so consecutive lanes store
 // consecutive addresses of one fine bucket's run: the pieces are a few dozen
-// bytes, and their half-written lines bound it (50 Mbp job: 520 -> 367 us for
-// 1.37 GB, 3.7 TB/s).  The running base of every
+// bytes, and their half-written lines bound it (50 Mbp job: 520 -> 367 us, 1.94 ->
+// 1.40 GB, 3.8 TB/s).  The running base of every
 // fine bucket carries from round to round, so the histogram holds one row per
 // planned tile (not one per round), and the next round's
 // slots are loaded while the current one is ranked.
@@ -2283,7 +2283,7 @@ __host__ __device__ constexpr uint32_t ct_tile(uint64_t m)
 // edges are written.  Contraction follows records; the home copies' own links
 // still hold their run heads and are spliced when something reads links
 // (k_splice_links): the fourth random access per pair took a quarter of the
-// kernel (50 Mbp job: 210 -> 152 us, all random lines).
+// kernel (50 Mbp job: 210 -> 152 us, 0.82 GB of random lines read, 0.08 written).
 __global__ __launch_bounds__(BLOCK) void k_splice(const uint32_t *__restrict__ pair_home,
                                                   const uint32_t *__restrict__ pair_borrow, uint32_t x,
                                                   const uint32_t *__restrict__ link, uint64_t *__restrict__ rec)
@@ -2379,7 +2379,7 @@ __device__ __forceinline__ uint64_t mlist_entry(uint32_t off, bool multi, uint32
 // thread takes one walk and all of a tile's chains of random reads are in
 // flight at once (with each thread walking its own slots one after another a
 // wave followed 2-3 walks at a time, eight times).  50 Mbp job: 310 -> 147 us,
-// bound by the latency of the walks' reads.
+// bound by the walks' random lines (0.82 GB read, 5.7 TB/s).
 template <int CT>
 __global__ __launch_bounds__(CT_NT) void k_seg_count(const uint64_t *__restrict__ rec, const uint32_t *__restrict__ hasp,
                                                      const uint8_t *__restrict__ flags, uint32_t m, uint32_t salt,
@@ -2913,7 +2913,7 @@ constexpr uint32_t emit_stage() { return W == 1 ? 2560 : 4608; }
 
 // Per tile: the live heads are gathered in slot order (39% of the slots:
 // walking the slots themselves left 61% of every wave's lanes idle through the
-// spelling, 0.85 ms on the 50 Mbp job, 0.51 so: 2.45 GB at 4.7 TB/s, what a
+// spelling, 0.85 ms on the 50 Mbp job, 0.52 so: 2.57 GB at 4.9 TB/s, what a
 // copy reaches), a scan of their lengths gives their text offsets, and the wave takes 64 of them at a time: one contiguous text
 // range, spelled into its LDS stage (put_kmer_lds, put_rest) and
 // written as aligned 16-byte lines, or straight to HBM when it does not fit.
