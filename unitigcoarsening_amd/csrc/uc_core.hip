@@ -5023,7 +5023,7 @@ int prepare_edges(uc_ctx *c)
         CHK(h2d(c, c->tcap.p, c->et_cap.data(), NF * 4));
     }
     CHK(ensure(c, c->table, total * sizeof(TEntry)));
-    CHK(ensure(c, c->hit, c->m * 4));
+    CHK(ensure(c, c->hit, NF ? c->m * 4 : 0));  // (the HBM tables' alone)
     CHK(ensure(c, c->link, c->m * 4));
     CHK(ensure(c, c->hasp, (c->m + 31) / 32 * 4 + 8));
     CHK(ensure(c, c->rec, c->m * 8 + 16));
