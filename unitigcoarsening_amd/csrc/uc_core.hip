@@ -4730,6 +4730,12 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         CHK(drop(c, c->src2));
         CHK(drop(c, c->perm));
         CHK(drop(c, c->hist2));
+        // and its plan
+        CHK(drop(c, c->tiles2));
+        CHK(drop(c, c->cbhb));
+        CHK(drop(c, c->cbts));
+        CHK(drop(c, c->cbtf));
+        CHK(drop(c, c->colsum));
     }
     c->l = l;
     c->bucketed = true;
@@ -5031,6 +5037,7 @@ int prepare_edges(uc_ctx *c)
     // has-predecessor bits: every bucket sets only its own slots' bits
     if (!c->hasp_clear) CHK(fill<uint32_t>(c, P<uint32_t>(c->hasp), (c->m + 31) / 32, 0u));
     c->hasp_clear = false;
+    CHK(drop(c, c->over));  // (read above)
     c->n_fallback = NF;
     c->n_groups = F;
     c->bucket_done.assign(G, 0);
@@ -5385,7 +5392,7 @@ int ensure_contraction(uc_ctx *c)
     CHK(ensure(c, c->ulen, c->m * 4));
     CHK(ensure(c, c->chainA, c->m * 8));
     CHK(ensure(c, c->chainB, c->m * 8));
-    CHK(ensure(c, c->list, c->m * 4));
+    CHK(ensure(c, c->list, c->n * 4));  // (run heads are home copies: one per k-mer at most)
     CHK(ensure(c, c->tsum, (T + 1) * 8));
     return UC_OK;
 }
