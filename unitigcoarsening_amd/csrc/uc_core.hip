@@ -2316,18 +2316,6 @@ __global__ void k_splice_links(const uint32_t *__restrict__ pair_home, const uin
     if (i < x) link[pair_home[i]] = link[pair_borrow[i]];
 }
 
-// list index for every flagged lane: one atomic per wave
-__device__ __forceinline__ uint32_t wave_append(bool flag, uint32_t *counter)
-{
-    const uint64_t bal = __ballot(flag);
-    if (!bal) return NONE;
-    const int leader = __builtin_ctzll(bal);
-    uint32_t base = 0;
-    if (__lane_id() == (uint32_t)leader) base = atomicAdd(counter, (uint32_t)__popcll(bal));
-    base = __shfl(base, leader, 64);
-    return base + (uint32_t)__popcll(bal & ((1ull << __lane_id()) - 1ull));
-}
-
 // counters in the context's small buffer
 // (uint32 indices: one 128-byte line each, so that atomics on different
 // counters never share a line; C_TOT holds two uint64 totals)
