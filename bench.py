@@ -15,7 +15,7 @@ from the warmup steps, where every launch is timed.  cpu_baseline =
 the serial restatement of the reference pipeline (oracle/refpipe.c) on a
 bounded sample of the same model, on one host core, checked against the
 GPU's output for that sample.  Beside it: "plain" (the same job with one
-shared table), "sets" (256 uneven sets, batched form vs per-set plain
+launch per bucket), "sets" (256 uneven sets, batched form vs per-set plain
 runs, both from HBM) and "serve" (the request loop under Poisson arrivals:
 p50 / p99 latency and k-mers/s).
 """
@@ -308,7 +308,7 @@ def bench_sets(args, keep=None):
             "batched_value": n / batched, "plain_value": n / plain, "batched_over_plain": round(plain / batched, 3),
             "texts_byte_equal": f"{equal} of {len(sizes)} sets",
             "note": "inputs resident in HBM for both forms; the plain form runs uc_compact per set on device "
-                    "pointers; after timing, every set's batched text is compared "
+                    "pointers with one launch per bucket; after timing, every set's batched text is compared "
                     "byte for byte with its plain run"}
 
 

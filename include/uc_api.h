@@ -43,9 +43,8 @@ extern "C" {
 
 /* bucket modes of the edge-finding phase */
 #define UC_MODE_BATCHED 0 /* one launch per phase over every bucket (and every set) */
-#define UC_MODE_PLAIN 1   /* one shared table sized for the largest bucket, which the buckets that
-                             need it take in turn, like the reference's per-bucket loop
-                             (driver.cpp:479-521); what fits LDS shares launches as above */
+#define UC_MODE_PLAIN 1   /* one launch per bucket, one shared table sized for the largest
+                             bucket, like the reference's per-bucket loop (driver.cpp:479-521) */
 
 typedef struct uc_ctx uc_ctx;
 

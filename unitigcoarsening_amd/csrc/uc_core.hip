@@ -4433,7 +4433,8 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
         // longer pieces of each fine bucket per round, and the buckets still
         // fit LDS groups (50 Mbp job: 512 instead of 1024 fine buckets per
         // coarse bucket, 3.91 against 3.96 ms per step on MI355X).  The plain
-        // form keeps the count, and with it the order of its lines.
+        // form keeps the count (its per-bucket launches measured 5.81 against
+        // 5.31 ms with the fewer, fuller fine buckets).
         if (!c->opts.fine_slots && want > MAX_SUB && c->opts.mode != UC_MODE_PLAIN)
             while (sub > 1 && ns * 112 / 100 <= (uint64_t)B * (sub / 2) * FINE_CAPPED_MAX) sub >>= 1;
         c->set_sub[s] = sub;
@@ -4869,14 +4870,16 @@ int prepare_edges(uc_ctx *c)
     const uint32_t load = c->opts.load_pct ? c->opts.load_pct : 50;
     const bool plain = c->opts.mode == UC_MODE_PLAIN;
     const uint32_t group_max = c->opts.group_slots ? c->opts.group_slots : LDS_GROUP;
-    // Fine buckets are packed to fewer slots when the launch would otherwise have
+    // Fine buckets are packed to fewer slots when a launch would otherwise have
     // under two groups per CU: a group's phases are a serial chain of barriers
     // and LDS round trips (24 us at 2048 slots), and small groups of it run
-    // side by side (60 k k-mers: 27 us in groups of 2048 slots, 14 in groups of
-    // 256).  1024 or 2048 groups as the line: the edge phase of 1 M k-mers 44 ->
-    // 50 and 53 us.
+    // side by side (1 M k-mers in 16 plain launches: 27 us each in groups of
+    // 2048 slots, 14 in groups of 256).  512 groups as the line: 256 and 1024
+    // measure the same there, and 1 M k-mers in one launch take 44 us of edge
+    // finding with it, 50 and 53 with 1024 and 2048.
     uint32_t group_pack = group_max;
-    while (group_pack > GROUP_PACK_MIN && c->n / group_pack < GROUPS_WANTED) group_pack /= 2;
+    const uint64_t per_launch = plain ? c->n / ((uint64_t)c->n_sets * c->B) : c->n;
+    while (group_pack > GROUP_PACK_MIN && per_launch / group_pack < GROUPS_WANTED) group_pack /= 2;
     const uint64_t F = c->cb_first[G];
     // groups planned on the device in one dense list: coarse bucket g's
     // groups are entries [gfirst[g], gfirst[g + 1])
@@ -5056,21 +5059,27 @@ int run_edges(uc_ctx *c, uint32_t bucket)
     const bool fresh = !c->edges_ready;  // planning clears the bitmap and the probe counters itself
     CHK(prepare_edges(c));
     const uint64_t G = (uint64_t)c->n_sets * c->B;
+    const bool plain = c->opts.mode == UC_MODE_PLAIN;
     if (bucket == UC_ALL_BUCKETS) {
         c->spliced = false;
         if (!fresh) {
             CHK(fill<uint32_t>(c, P<uint32_t>(c->hasp), (c->m + 31) / 32, 0u));
             CHK(clear_probes(c));
         }
-        // groups and slices share nothing between buckets, so the plain form
-        // too takes all of a job's in one launch; its buckets take turns
-        // (driver.cpp:479-521) only at the HBM table that they share.  (1 M
-        // k-mers in 16 buckets: 16 launches of 8 us against one of 25, the phase 146
-        // against 44 us.)
-        CHK(launch_lds_edges<W>(c, 0, c->grp_first[G]));
-        CHK(launch_big_edges<W>(c, 0, c->bg_first[G]));
-        CHK(launch_slice_edges<W>(c, 0, c->sl_first[G]));
-        CHK(run_fallback<W>(c, 0, c->fb_first[G]));
+        if (!plain) {
+            CHK(launch_lds_edges<W>(c, 0, c->grp_first[G]));
+            CHK(launch_big_edges<W>(c, 0, c->bg_first[G]));
+            CHK(launch_slice_edges<W>(c, 0, c->sl_first[G]));
+            CHK(run_fallback<W>(c, 0, c->fb_first[G]));
+        } else {
+            // the reference's per-bucket loop (driver.cpp:479-521)
+            for (uint64_t g = 0; g < G; g++) {
+                CHK(launch_lds_edges<W>(c, c->grp_first[g], c->grp_first[g + 1] - c->grp_first[g]));
+                CHK(launch_big_edges<W>(c, c->bg_first[g], c->bg_first[g + 1] - c->bg_first[g]));
+                CHK(launch_slice_edges<W>(c, c->sl_first[g], c->sl_first[g + 1] - c->sl_first[g]));
+                CHK(run_fallback<W>(c, c->fb_first[g], c->fb_first[g + 1]));
+            }
+        }
         std::fill(c->bucket_done.begin(), c->bucket_done.end(), 1);
         c->n_done = G;
     } else {
