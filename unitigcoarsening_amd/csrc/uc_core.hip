@@ -5177,8 +5177,10 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
     uint32_t *cnt = P<uint32_t>(c->small);
     const uint32_t *np = cnt + C_LIST;
     uint64_t *ca = P<uint64_t>(c->chainA), *cb = P<uint64_t>(c->chainB);
-    // small jobs rank their chains in one workgroup
-    const bool one = spec && T <= CHAIN_ONE_TILES && (m >> c->shift) <= CHAIN_ONE_LIST;
+    // small jobs rank their chains in one workgroup, where its LDS holds the tile sums
+    const size_t one_lds = T * 8 + 1024;
+    const bool one = spec && T <= CHAIN_ONE_TILES && (m >> c->shift) <= CHAIN_ONE_LIST &&
+                     one_lds <= c->lds_limit;
     // (the bucketing cleared the counters of a small job's first pass)
     const bool cleared = one && c->cnt_clear;
     c->cnt_clear = false;
@@ -5206,7 +5208,7 @@ int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true
     auto spec_pass = [&]() -> int {
         CHK(walks());
         if (one) {
-            CHK(allow_lds(c, k_chain_one, T * 8 + 1024));
+            CHK(allow_lds(c, k_chain_one, one_lds));
             KLAUNCH(c, "k_chain_one", k_chain_one, (1, CHAIN_ONE_NT, T * 8), P<uint32_t>(c->list), cnt,
                     P<uint32_t>(c->hasp), P<uint32_t>(c->prevseg), P<uint64_t>(c->seg), ca, cb, P<uint32_t>(c->ulen),
                     P<uint64_t>(c->tsum), P<uint64_t>(c->tcnt), (uint32_t)T, ct);
@@ -5773,6 +5775,13 @@ int uc_ctx_set_slice_probes(uc_ctx *c, uint32_t probes)
 {
     if (!c || probes < 1 || probes > SLICE_TAB) return UC_E_ARG;
     c->slice_probes = probes;
+    return UC_OK;
+}
+
+int uc_ctx_set_lds_limit(uc_ctx *c, uint32_t bytes)
+{
+    if (!c || bytes < 65536 || bytes > c->lds_limit) return UC_E_ARG;
+    c->lds_limit = bytes;
     return UC_OK;
 }
 

@@ -1,5 +1,6 @@
 // uc_internal.h -- library-internal hooks between the compaction contexts
-// (uc_core.hip) and the request loop (uc_server.cpp).  Not part of the C ABI.
+// (uc_core.hip), the request loop (uc_server.cpp) and the tests.  Not part of
+// the C ABI.
 #pragma once
 #include <stdint.h>
 
@@ -41,3 +42,8 @@ int uc_text_copy_pinned(uc_ctx *c, char *dst, uint64_t cap);
 // DMA engine, so that they overlap the copies of other contexts sharing the
 // device.  Call from the context's own thread.
 void uc_ctx_set_kernel_copies(uc_ctx *c, bool on);
+
+// LDS that the context's kernels may take per workgroup, from 64 KiB to what
+// it has now (the device's): a job takes the routes of a device with that
+// much.  For tests.
+extern "C" int uc_ctx_set_lds_limit(uc_ctx *c, uint32_t bytes);
