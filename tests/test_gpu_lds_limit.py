@@ -9,8 +9,9 @@ import unitigcoarsening_amd as uc
 pytestmark = pytest.mark.gpu
 
 
-# 4.3 M k-mers: more tile sums than 64 KiB hold
-@pytest.mark.parametrize("k,n,opts", [(31, 4_300_000, {}), (63, 4_300_000, {})])
+# 4.3 M k-mers: more tile sums than 64 KiB hold.  2.5 M in 64 buckets of 16 fine buckets: 1024 rows in one pass, whose
+# counters are 74 KB.
+@pytest.mark.parametrize("k,n,opts", [(31, 4_300_000, {}), (63, 4_300_000, {}), (31, 2_500_000, {"fine_slots": 4096})])
 def test_small_lds(k, n, opts):
     kmers = uc.medium_model(23, n + n // 16, k)[:n]
     limit = uc.lib().uc_ctx_set_lds_limit

@@ -4441,19 +4441,21 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     }
     const bool keep_src = (c->opts.flags & UC_FLAG_KEEP_SRC) != 0;
     c->tile2 = 0;
-    // how the fine bits are split over the two passes (see split_bits)
-    const uint32_t nb = (uint32_t)__builtin_ctz(B);
-    uint32_t smax = 1;
-    for (uint32_t sb : c->set_sub) smax = std::max(smax, sb);
-    const uint32_t J = pass1_fine_bits(nb, (uint32_t)__builtin_ctz(smax), S);
-    const uint32_t R = B << J;                                    // pass-1 rows per set
-    const uint32_t s1max = std::max(smax >> J, 1u);               // most fine buckets of a row
-    const bool any_fine = s1max > 1;                              // a second pass follows
     // k-mers per bucketing tile: small jobs take small ones, so that they
     // spread over the CUs
     constexpr uint32_t TILE1 = (W == 1 ? 8 : 4) * BLOCK, TILE1_SMALL = 512;
     const uint32_t tile1 = c->n <= TILE1_SMALL_MAX ? TILE1_SMALL : TILE1;
     c->tile1 = tile1;
+    // how the fine bits are split over the two passes (see split_bits)
+    const uint32_t nb = (uint32_t)__builtin_ctz(B);
+    uint32_t smax = 1;
+    for (uint32_t sb : c->set_sub) smax = std::max(smax, sb);
+    uint32_t J = pass1_fine_bits(nb, (uint32_t)__builtin_ctz(smax), S);
+    // (64 KiB of LDS per workgroup hold the counters of 512 rows in large tiles)
+    while (J && lmin_lds_bytes(B << J, tile1 / 64) > c->lds_limit) J--;
+    const uint32_t R = B << J;                                    // pass-1 rows per set
+    const uint32_t s1max = std::max(smax >> J, 1u);               // most fine buckets of a row
+    const bool any_fine = s1max > 1;                              // a second pass follows
     // tiles: every set gets at least one (possibly empty) tile so each bucket
     // row has a start in the histogram; the tiles are filled on the device
     std::vector<uint64_t> set_plan(3 * (uint64_t)S + 2);  // set offsets, tile prefix, then the sets' fine counts
