@@ -2270,9 +2270,10 @@ constexpr int CT_NT = 64;
 constexpr uint32_t CT_MIN = 64, CT_MAX = 512;
 static_assert(CT_MAX <= 2048, "a tile's list entries hold slot offsets in 11 bits");
 
-__host__ __device__ constexpr uint32_t ct_tile(uint64_t m)
+// A job that has to be frugal with memory takes the largest.
+__host__ __device__ constexpr uint32_t ct_tile(uint64_t m, bool frugal)
 {
-    uint32_t t = CT_MIN;
+    uint32_t t = frugal ? CT_MAX : CT_MIN;
     while (t < CT_MAX && (m + t - 1) / t > (uint64_t)SCAN_TILE) t *= 2;
     return t;
 }
@@ -3393,6 +3394,7 @@ struct uc_ctx {
     bool lazy_sizes = false, sizes_pending = false;
     // the bucketing has cleared the predecessor bits / the counters already
     bool hasp_clear = false, cnt_clear = false;
+    bool frugal = false;  // the budget may not hold what small tiles take beyond large ones
     bool timed = false;  // emission records the job's last phase boundary
     char *pin[2] = {nullptr, nullptr};
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
@@ -4444,7 +4446,10 @@ int run_bucketize(uc_ctx *c, uint32_t l, const uint32_t *table)
     // k-mers per bucketing tile: small jobs take small ones, so that they
     // spread over the CUs
     constexpr uint32_t TILE1 = (W == 1 ? 8 : 4) * BLOCK, TILE1_SMALL = 512;
-    const uint32_t tile1 = c->n <= TILE1_SMALL_MAX ? TILE1_SMALL : TILE1;
+    // (not under a budget below the most that the job can need: small tiles
+    // have more histogram rows, up to 3% of a job with 1024 buckets)
+    c->frugal = c->opts.hbm_budget && c->opts.hbm_budget < uc_job_bytes_estimate(c->n, c->k);
+    const uint32_t tile1 = c->n <= TILE1_SMALL_MAX && !c->frugal ? TILE1_SMALL : TILE1;
     c->tile1 = tile1;
     // how the fine bits are split over the two passes (see split_bits)
     const uint32_t nb = (uint32_t)__builtin_ctz(B);
@@ -5174,7 +5179,7 @@ int with_ct(uint32_t ct, F f)
 int contract_pass(uc_ctx *c, uint64_t *live, uint32_t *nonconv, bool spec = true, bool defer = false)
 {
     const uint32_t m = (uint32_t)c->m;
-    const uint32_t ct = ct_tile(c->m);
+    const uint32_t ct = ct_tile(c->m, c->frugal);
     const uint64_t T = (c->m + ct - 1) / ct;
     uint32_t *cnt = P<uint32_t>(c->small);
     const uint32_t *np = cnt + C_LIST;
@@ -5383,7 +5388,8 @@ int cut_cycles(uc_ctx *c, uint64_t *n_cut)
 // every array a contraction pass writes or reads besides the edge result
 int ensure_contraction(uc_ctx *c)
 {
-    const uint64_t T = (c->m + ct_tile(c->m) - 1) / ct_tile(c->m);
+    const uint32_t ct = ct_tile(c->m, c->frugal);
+    const uint64_t T = (c->m + ct - 1) / ct;
     CHK(ensure(c, c->small, C_WORDS * 4));
     CHK(ensure(c, c->tcnt, (T + 1) * 8));
     CHK(ensure(c, c->seg, c->m * 8));
@@ -5493,7 +5499,7 @@ template <int W>
 int run_emit(uc_ctx *c)
 {
     const uint32_t m = (uint32_t)c->m;
-    const uint32_t ct = ct_tile(c->m);
+    const uint32_t ct = ct_tile(c->m, c->frugal);
     const uint64_t T = (c->m + ct - 1) / ct;
     if (c->text_fixed) {
         // the caller's buffer (uc_compact_noalloc); the kernels write bytes [0, text_bytes) only
