@@ -1375,13 +1375,12 @@ __global__ __launch_bounds__(NT) void k_sub_scatter(const BTile *__restrict__ ti
                 M = match_bit(M, lanes_of(m != 0), m);
             }
             // the wave's base in the bucket moves past the group (its last lane
-            // writes it; a wave's LDS accesses keep their order)
+            // writes it)
             const uint32_t rank = below(M, 0), size = (uint32_t)__popcll(M);
             uint32_t base = 0;
-            if (valid) {
-                base = mywc[v];
-                if (rank + 1 == size) mywc[v] = base + size;
-            }
+            if (valid) base = mywc[v];
+            wave_sync();  // every lane of the group has read it
+            if (valid && rank + 1 == size) mywc[v] = base + size;
             wave_sync();
             if (valid) {
                 const uint64_t s = t.kbegin + r0 + c0 + 64u * j + (uint32_t)lane;
