@@ -4022,26 +4022,27 @@ int staged_d2h(uc_ctx *c, void *dst_, const void *src_, uint64_t bytes)
     CHK(stage_pinned(c));
     const uint64_t np = (bytes + STAGE_STEP - 1) / STAGE_STEP;
     const int T = (int)std::min<uint64_t>(COPY_THREADS, np), dev = c->opts.device;
-    std::atomic<bool> bad{false};
+    std::atomic<int> err{hipSuccess};  // the first error of any thread
+    auto ok = [&](hipError_t e) {
+        int none = hipSuccess;
+        if (e != hipSuccess) err.compare_exchange_strong(none, e);
+        return e == hipSuccess;
+    };
     auto len = [&](uint64_t i) { return std::min<uint64_t>(STAGE_STEP, bytes - i * STAGE_STEP); };
     auto worker = [&](int t) {
-        if (hipSetDevice(dev) != hipSuccess) bad = true;
+        if (!ok(hipSetDevice(dev))) return;
         auto piece = [&](uint64_t r) { return (uint64_t)t + r * (uint64_t)T; };
         auto dma = [&](uint64_t r) {
             const uint64_t i = piece(r), off = i * STAGE_STEP;
             const int b = 2 * t + (int)(r & 1);
-            if (hipMemcpyAsync(c->spin[b], src + off, len(i), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-                hipEventRecord(c->spin_ev[b], c->stream) != hipSuccess)
-                bad = true;
+            return ok(hipMemcpyAsync(c->spin[b], src + off, len(i), hipMemcpyDeviceToHost, c->stream)) &&
+                   ok(hipEventRecord(c->spin_ev[b], c->stream));
         };
-        if (!bad) dma(0);
-        for (uint64_t r = 0; piece(r) < np && !bad; r++) {
+        if (!dma(0)) return;
+        for (uint64_t r = 0; piece(r) < np && err == hipSuccess; r++) {
             const int b = 2 * t + (int)(r & 1);
-            if (piece(r + 1) < np) dma(r + 1);  // into the other piece, copied out already
-            if (bad || hipEventSynchronize(c->spin_ev[b]) != hipSuccess) {
-                bad = true;
-                break;
-            }
+            if (piece(r + 1) < np && !dma(r + 1)) return;  // into the other piece, copied out already
+            if (!ok(hipEventSynchronize(c->spin_ev[b]))) return;
             std::memcpy(dst + piece(r) * STAGE_STEP, c->spin[b], len(piece(r)));
         }
     };
@@ -4059,7 +4060,9 @@ int staged_d2h(uc_ctx *c, void *dst_, const void *src_, uint64_t bytes)
     for (int t = 1; t < T; t++)
         if (th[t].joinable()) th[t].join();
     // (the pieces are free again for the next copy once the stream is idle)
-    if (hipStreamSynchronize(c->stream) != hipSuccess || bad) return fail(c, UC_E_HIP, "staged copy");
+    (void)ok(hipStreamSynchronize(c->stream));
+    if (err != hipSuccess)
+        return fail(c, UC_E_HIP, std::string("copying the text out: ") + hipGetErrorString((hipError_t)err.load()));
     return UC_OK;
 }
 
