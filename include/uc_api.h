@@ -302,7 +302,8 @@ typedef struct {
 } uc_timing;
 
 /* Per-phase device times (HIP events on the context's stream) of the last
- * uc_compact / uc_compact_sets. */
+ * uc_compact / uc_compact_sets.  emit_ms and total_ms end with the job's last
+ * kernel: the host's read of the totals after it (about 10 us) is in neither. */
 int uc_timing_get(uc_ctx *ctx, uc_timing *t);
 
 /* With UC_FLAG_PROFILE: accumulated device time and launch count of kernel

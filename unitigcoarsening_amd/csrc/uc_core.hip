@@ -602,8 +602,9 @@ __global__ __launch_bounds__(BLOCK) void k_lmin_count(const uint64_t *__restrict
     const uint32_t bmask = p.B - 1, nbits = (uint32_t)__builtin_ctz(p.B), s1 = t.split >> 16;
     // the order's operands in vector registers: an instruction takes one scalar
     // register, and moves outside the inner loops brought the second (with the
-    // 32-bit reversal: 48 M 31-mers 271 -> 243 us, 206 instructions per k-mer,
-    // which alone are 252 us at full issue; 140 M 63-mers 1897 -> 1694 us)
+    // 32-bit reversal: 48 M 31-mers 271 -> 243-257 us, 207 vector instructions
+    // per k-mer issued at one per CU and cycle or a little more, which bounds
+    // it; 140 M 63-mers 1897 -> 1694 us)
     asm("" : "+v"(p.k1), "+v"(p.w1), "+v"(p.w2));
     // all of this thread's k-mers in flight at once (threads past the end load
     // the last one: a branch per item would wait for each load in turn)
@@ -767,8 +768,10 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t *a, uint32_t n, uin
 // one bucket); per wave the rank among placements bound for the same bucket
 // comes from matching the bucket number bit by bit (match_bit).  Every thread's
 // codes and k-mers are loaded up front, so all of them are in flight at once.
-// (48 M 31-mers: 550 us with an array of lane masks per bit, 300 so; 226
-// instructions per k-mer, 276 us of them, bound it, not its 1.2 GB.)  With
+// (48 M 31-mers: 550 us with an array of lane masks per bit, 300-330 so; 226
+// vector instructions per k-mer, 0.9 per CU and cycle, bound it, not its
+// 1.2 GB.  At 300 M 63-mers, 0.6 per CU and cycle and 13 GB at 3.7 TB/s:
+// neither alone.)  With
 // STAGE, the tile's placements are gathered in LDS in bucket order and leave
 // as runs of consecutive slots; a tile with more placements than the stage
 // holds (more than a quarter of its k-mers crossing) stores them directly.
@@ -1859,9 +1862,10 @@ __global__ __launch_bounds__(PLAN_ONE_NT) void k_plan_one(const uint32_t *__rest
 // Keys of different fine buckets never match (equal (k-1)-mers have
 // equal minimizers), so a group shares one table.  HBM sees only the
 // sequential k-mer/flag reads and link writes plus one bitmap word per 32
-// slots.  Instructions bound it (50 Mbp job: 321 per slot, 431 of its 499 us,
-// 790 before the probe loops had one exit, the hash one multiply fewer and the
-// hits stayed in registers); its 1.0 GB would take 220 us.
+// slots.  Instructions bound it (50 Mbp job: 322 vector instructions per slot,
+// 0.9 per CU and cycle; 500 us, 790 before the probe loops had one exit, the
+// hash one multiply fewer and the hits stayed in registers); its 1.0 GB would
+// take 220 us.
 //   LDS layout (nb = launch capacity, a power of two):
 //     km   Kmer<W>[nb]   staged k-mers
 //     tab  uint32[2nb]   owner (16 bits) | LDS_SHARED | hits << 24, or LDS_EMPTY
