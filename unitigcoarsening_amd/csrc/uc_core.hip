@@ -3158,6 +3158,12 @@ __global__ void k_link_succ(const uint32_t *__restrict__ link, const uint8_t *__
 constexpr uint32_t TXT_TILE = BLOCK * 16;
 constexpr uint32_t TXT_PAD = TXT_TILE + 256;
 
+// bit 7 of every byte of x that is zero
+__device__ __forceinline__ uint32_t zero_bytes(uint32_t x)
+{
+    return ~(((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x | 0x7F7F7F7Fu);
+}
+
 // bit b set iff byte b of the 16 at `pos` is '\n' and lo <= pos + b < hi
 __device__ __forceinline__ uint32_t nl_mask16(uint4 v, uint64_t pos, uint64_t lo, uint64_t hi)
 {
@@ -3165,8 +3171,7 @@ __device__ __forceinline__ uint32_t nl_mask16(uint4 v, uint64_t pos, uint64_t lo
     uint32_t m = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const uint32_t t = w[j] ^ 0x0A0A0A0Au;  // zero bytes where '\n'
-        const uint32_t z = ~(((t & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | t | 0x7F7F7F7Fu);  // 0x80 per zero byte
+        const uint32_t z = zero_bytes(w[j] ^ 0x0A0A0A0Au);  // 0x80 per '\n'
         const uint32_t nib = ((z >> 7) & 1u) | ((z >> 14) & 2u) | ((z >> 21) & 4u) | ((z >> 28) & 8u);
         m |= nib << (4 * j);
     }
@@ -3197,9 +3202,8 @@ __device__ __forceinline__ uint32_t txt_code(char ch)
 // word the codes from two bits of each character, the characters those codes
 // stand for (one byte permute) to compare with, and one multiply that gathers
 // the four codes in its top byte.  Byte by byte a line waited for 31 loads in a
-// row: 2 M 31-mers (64 MB) took 164 us, this way 32.  Any other byte, and a line
-// that ends early, is left to the loop below.  The text has TXT_PAD bytes after
-// its end.
+// row: 2 M 31-mers (64 MB) took 164 us, this way 32.  The text has
+// TXT_PAD bytes after its end.
 template <int W>
 __device__ __forceinline__ bool pack_acgt(const char *__restrict__ txt, uint64_t start, uint32_t k, uint64_t *w)
 {
@@ -3225,6 +3229,42 @@ __device__ __forceinline__ bool pack_acgt(const char *__restrict__ txt, uint64_t
     return bad == 0;
 }
 
+// The same for a line with other bytes, which count as A, when it does not end
+// within the k bytes nor may (a '\r' as the k-th): 16 bytes at a time, in a
+// rolled loop that leaves the registers and the code to pack_acgt.  (Byte by byte
+// after pack_acgt such lines took longer than byte by byte alone: 2 M 63-mers
+// in lower case 550 -> 653 us; this way 156 us.)
+template <int W>
+__device__ __forceinline__ bool pack_any(const char *__restrict__ txt, uint64_t len, uint64_t start, uint32_t k,
+                                         uint64_t *w)
+{
+    if (start + k > len) return false;
+    uint32_t ends = txt[start + k - 1] == '\r';
+    w[0] = w[W - 1] = 0;
+#pragma unroll 1
+    for (uint32_t b = 0; b < k; b += 16) {
+        uint4 v;
+        __builtin_memcpy(&v, txt + start + b, 16);
+        const uint32_t x4[4] = {v.x, v.y, v.z, v.w};
+        uint32_t codes = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t at = b + 4 * j;
+            // (bytes past the k-th count as A)
+            const uint32_t keep = at + 4 <= k ? ~0u : at < k ? (1u << (8 * (k - at))) - 1u : 0u;
+            const uint32_t x = (x4[j] & keep) | (0x41414141u & ~keep), c = ((x >> 1) ^ (x >> 2)) & 0x03030303u;
+            const uint32_t same = zero_bytes(__builtin_amdgcn_perm(0u, 0x54474341u, c) ^ x) >> 7;
+            ends |= zero_bytes(x ^ 0x0A0A0A0Au);
+            codes |= (((c & (same * 3u)) * 0x01041040u) >> 24) << (8 * j);
+        }
+        if (W == 1 || b < 32)
+            w[0] |= (uint64_t)codes << (2 * b);
+        else
+            w[W - 1] |= (uint64_t)codes << (2 * b - 64);
+    }
+    return ends == 0;
+}
+
 // line `idx` starting at `start`: its first k characters, or an error when
 // the line (without one '\r' before its end) is shorter than k
 template <int W>
@@ -3232,7 +3272,7 @@ __device__ __forceinline__ void pack_line(const char *__restrict__ txt, uint64_t
                                           uint32_t k, uint64_t *__restrict__ out, uint32_t *__restrict__ err)
 {
     uint64_t w[2] = {0, 0};
-    if (pack_acgt<W>(txt, start, k, w)) {
+    if (pack_acgt<W>(txt, start, k, w) || pack_any<W>(txt, len, start, k, w)) {
 #pragma unroll
         for (int j = 0; j < W; j++) out[idx * W + j] = w[j];
         return;
